@@ -11,9 +11,12 @@
 //
 // Backward: one block per tile, dispatched heaviest tile first, replays the
 // tile's list back-to-front from its largest last_id, rebuilding
-// transmittance per pixel; per record, a wave sums its lanes' partial
-// gradients by a transposed DPP/permlane reduction into per-wave LDS slots,
-// and each batch ends with one atomic per (record, nonzero component).
+// transmittance per pixel, and each batch ends with one atomic per (record,
+// nonzero component). raster_bwd_rows_kernel (the training path) keeps 16
+// records in a wave's lanes and runs the pixel recurrences across them;
+// raster_bwd_kernel (other tile sides, more than four channels, absolute
+// gradients) keeps pixels in lanes and sums each record's partial gradients
+// over the wave by a transposed DPP/permlane reduction into per-wave LDS slots.
 //
 // Per-pixel math follows gsplat_core/gsplat_rasterize.cpp:291-368 (forward)
 // and :432-554 (backward) operation for operation; the Gaussian falloff and
@@ -24,6 +27,7 @@
 #include <atomic>
 #include <climits>
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "scan.hpp"
@@ -118,6 +122,47 @@ __device__ __forceinline__ float exp_alpha(float y) {
   const float n = __builtin_rintf(ph);
   const float f = (ph - n) + pl;
   return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+}
+
+// exp_alpha for y in (-2.98e9, 0], bit for bit, without the lower clamp.
+__device__ __forceinline__ float exp_alpha_bounded(float y) {
+  const float head = 1.44269502162933349609375f;  // float(log2 e)
+  const float tail = __uint_as_float(0x32a5705fu);
+  const float ph = y * head;
+  float pl = __builtin_fmaf(y, head, -ph);
+  pl = __builtin_fmaf(y, tail, pl);
+  const float n = __builtin_rintf(ph);
+  const float f = (ph - n) + pl;
+  return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+}
+
+// Classes of records whose alpha needs fewer tests for the same result
+// (staged with the record's touch mask, bits above the waves'):
+// - kGeneralRecord clear: a conic well inside the positive definite ones
+//   (det > 1e-4 c0 c2 keeps the computed sigma >= 0: its rounding is below
+//   1e-6 of c0 dx^2 + c2 dy^2, the form above 5e-5 of it, and neither
+//   underflows), and an opacity up to 1. A visiting wave has a pixel with
+//   sigma below 6 within 44 pixels of every other one, and c0 + c2 <= 2e6
+//   then keeps sigma below 2e9, so the exponential needs no clamp.
+// - kCappedRecord clear: also an opacity up to 0.99, so alpha = o exp(-sigma)
+//   never meets the cap.
+constexpr uint32_t kNonFiniteRecord = 1u << 31;  // a non-finite mean or staged colour (backward)
+constexpr uint32_t kGeneralRecord = 1u << 30;
+constexpr uint32_t kCappedRecord = 1u << 29;
+
+__device__ __forceinline__ uint32_t record_class(float2 m, float4 co) {
+  const bool plain = co.x > 1.0e-15f && co.z > 1.0e-15f && co.x < 1.0e6f && co.z < 1.0e6f &&
+                     co.x * co.z - co.y * co.y > 1.0e-4f * co.x * co.z && fabsf(m.x) < 1.0e9f &&
+                     fabsf(m.y) < 1.0e9f && co.w <= 1.0f;
+  if (!plain) return kGeneralRecord | kCappedRecord;
+  return co.w <= kMaxAlpha ? 0u : kCappedRecord;
+}
+
+// sigma of a record with a halved conic diagonal: (0.5 c0 dx) dx + (0.5 c2 dy) dy
+// equals 0.5 ((c0 dx) dx + (c2 dy) dy) bit for bit (scaling by 2 commutes with
+// rounding away from the subnormal range), one multiply less per visit.
+__device__ __forceinline__ float halved_sigma(const float4& co, float dx, float dy) {
+  return (co.x * dx * dx + co.z * dy * dy) + co.y * dx * dy;
 }
 
 // ---------------------------------------------------------------------------
@@ -265,10 +310,6 @@ __device__ __forceinline__ uint32_t touch_mask(float2 m, float4 co, int n_waves,
 // Words of one forward batch record in LDS: conic xyz + opacity, then mean xy
 // and the CH staged colours (CH == 0: the Gaussian id), padded to 16 bytes.
 __host__ __device__ constexpr int fwd_record_words(int ch) { return 4 + (2 + (ch > 0 ? ch : 1) + 3) / 4 * 4; }
-// Touch-mask bit of a backward record whose mean or staged colours are not
-// all finite.
-constexpr uint32_t kNonFiniteRecord = 1u << 31;
-
 // CH in 1..4: colors staged in LDS; CH == 0: runtime channel count (<= 64),
 // colors read from global memory.
 //
@@ -540,8 +581,8 @@ __device__ __forceinline__ void wave_transpose_reduce(const float (&v)[N], float
 // to clear). CH == 0 (runtime channel count) sends colour gradients straight
 // to global memory.
 // Six waves per SIMD (at most 80 VGPRs) where that needs no spills: one to
-// three channels without absgrad (the training path); the register need
-// leaves the others as they are.
+// three channels without absgrad; the register need leaves the others as they
+// are.
 constexpr int bwd_min_waves(int ch, bool abs) { return (!abs && ch >= 1 && ch <= 3) ? 6 : 1; }
 // s_waitcnt immediate (gfx9 encoding): vmcnt 0 (bits 3:0 and 15:14), expcnt 7
 // (bits 6:4) and lgkmcnt 15 (bits 11:8), i.e. wait for vector memory only
@@ -934,6 +975,459 @@ raster_bwd_kernel(
   }
 }
 
+// Inclusive prefix product / sum over each row of 16 lanes, four independent
+// values at a time: DPP row shifts by 1, 2, 4, 8 in place, a lane without a
+// source keeps its value. The four chains are interleaved, so each DPP read
+// comes at least two wait states after the write it depends on (the s_nop
+// covers the values' producers).
+#define GSPLAT_ROW_STEP(OP, SH)                              \
+  OP " %0, %0, %0 row_shr:" SH " row_mask:0xf bank_mask:0xf\n\t" \
+  OP " %1, %1, %1 row_shr:" SH " row_mask:0xf bank_mask:0xf\n\t" \
+  OP " %2, %2, %2 row_shr:" SH " row_mask:0xf bank_mask:0xf\n\t" \
+  OP " %3, %3, %3 row_shr:" SH " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void row16_product4(float (&v)[4]) {
+  asm("s_nop 1\n\t" GSPLAT_ROW_STEP("v_mul_f32_dpp", "1") GSPLAT_ROW_STEP("v_mul_f32_dpp", "2")
+          GSPLAT_ROW_STEP("v_mul_f32_dpp", "4") GSPLAT_ROW_STEP("v_mul_f32_dpp", "8")
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+// v: inclusive sums; before: each lane's exclusive sum (the previous lane's
+// inclusive one), lane 0 of the row keeps the value it came with.
+__device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
+  asm("s_nop 1\n\t" GSPLAT_ROW_STEP("v_add_f32_dpp", "1") GSPLAT_ROW_STEP("v_add_f32_dpp", "2")
+          GSPLAT_ROW_STEP("v_add_f32_dpp", "4") GSPLAT_ROW_STEP("v_add_f32_dpp", "8")
+      "v_mov_b32_dpp %4, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %5, %1 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %6, %2 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %7, %3 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(before[0]), "+v"(before[1]), "+v"(before[2]),
+        "+v"(before[3]));
+}
+#undef GSPLAT_ROW_STEP
+
+// Backward with records in lanes: tiles whose side is a multiple of 8, one to
+// four channels, no absolute gradients (the training path). Block, schedule,
+// staging and flush are raster_bwd_kernel's; a wave still owns an 8x8 block of
+// pixels, but evaluates 16 records at a time: lane l holds record l % 16 of
+// the group (in list order, back to front) and the pixel rows l / 16 and
+// l / 16 + 4, and steps over the 8 columns.
+// - A record's gradient sums stay in its lane's registers over all the wave's
+//   pixels; one exchange over the four rows per group replaces a 64-lane
+//   reduction per record.
+// - The pixel recurrences run across the 16 lanes instead of over time: T is a
+//   prefix product of 1 / (1 - alpha) and the buffer a prefix sum, four DPP
+//   steps each; lane 0 brings the pixel's state in, lane 15 leaves it in LDS.
+// - A column's (0.5 c0 dx) dx and c1 dx serve both of the lane's rows, a
+//   row's (0.5 c2 dy) dy all eight columns; sigma keeps the forward's operations
+//   and rounding. Sums over y need no per-pixel products: with S and Hx the
+//   sums of v_sigma and v_sigma dx over one row, sum v_sigma dy = S dy.
+// - Groups without capped or general records (see above) skip the cap's and
+//   sigma's tests.
+// - The waves add their sums to one slot per entry in double (LDS atomics), so
+//   the order in which waves arrive does not show in the rounded result.
+//
+// - While entries remain before a batch, a wave evaluates whole groups only;
+//   the next batch starts at the first entry some wave left over (each wave
+//   skips what it has done). Groups then hold the same records whatever the
+//   tile's list holds beside them, so the same pixels' recurrences round the
+//   same with AABB and ellipse lists.
+//
+// Bound by VALU issue (0.98 of the issue slots at 1M Gaussians, 1297x840):
+// 46 instructions per 64 (pixel, record) evaluations and about 10 around them,
+// against 78 of the kernel with pixels in lanes. There 313 -> 231 us; 4.12 ->
+// 3.23 ms over 8 images of 1920x1080, 470 -> 343 us for large faint splats,
+// 114 -> 81 us at 512x512. About 120 VGPRs hold four evaluations in flight
+// (their scans interleave without wait states); at five waves per SIMD (96
+// VGPRs) the loop spills, 293 us, and unrolled further it does at four.
+// Batches of 256 entries (4 blocks per CU by LDS) measured 231 us, 192 243 us
+// and 128 246 us (without the carried-over groups).
+constexpr int kRowsBatch = 256;
+constexpr int kRowsAdvance = 128;  // a batch advances by at least this many entries
+constexpr int kNeutral = 40;  // entries of the neutral state: columns 0-7 of two rows 32 apart
+
+template <int CH>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) raster_bwd_rows_kernel(
+    RasterArgs a, int BB, int64_t n_units, const int32_t* __restrict__ order, const int32_t* __restrict__ cost,
+    const float* __restrict__ render_alphas, const int32_t* __restrict__ last_ids,
+    const float* __restrict__ v_render_colors, const float* __restrict__ v_render_alphas,
+    float* __restrict__ v_means2d, float* __restrict__ v_conics, float* __restrict__ v_colors,
+    float* __restrict__ v_opacities) {
+  constexpr int NV = CH + 6;
+  constexpr int NS = NV | 1;  // accumulator words per slot (odd: no bank conflicts between records)
+  constexpr int RW = bwd_record_words(CH);
+  constexpr int GW = 6 + CH;
+  extern __shared__ float smem[];
+  const int BS = blockDim.x;
+  const int n_waves = BS / kWave;
+  double* s_acc = reinterpret_cast<double*>(smem);                  // [BB][NS]
+  float4* s_pix = reinterpret_cast<float4*>(s_acc + BB * NS + (BB * NS & 1));  // [BS] colour cotangents (and last id)
+  float2* s_state = reinterpret_cast<float2*>(s_pix + BS);          // [BS] T, Bc
+  int* s_last = reinterpret_cast<int*>(s_state + BS);               // [BS]
+  float2* s_neutral = reinterpret_cast<float2*>(s_last + (CH == 4 ? BS : 0));  // [kNeutral] (1, 0)
+  float* s_rec = reinterpret_cast<float*>(s_neutral + kNeutral);          // [BB][RW]
+  float4* s_rect = reinterpret_cast<float4*>(s_rec + RW * BB);      // [n_waves]
+  int* s_next = reinterpret_cast<int*>(s_rect + n_waves);           // [n_waves]
+  uint16_t* s_list = reinterpret_cast<uint16_t*>(s_next + n_waves); // [n_waves][BB]
+  auto s_g = [&](int k) { return __float_as_int(s_rec[k * RW + GW]); };
+  auto s_mask = [&](int k) { return __float_as_uint(s_rec[k * RW + GW + 1]); };
+
+  const int t = threadIdx.x;
+  const int lane = t % kWave;
+  const int wave = t / kWave;
+  const int64_t n_tiles = static_cast<int64_t>(a.tw) * a.th;
+  // flush role of this thread (raster_bwd_kernel)
+  const int fc = t % kFlushLanes;
+  int fl_word0 = -1, fl_word1 = -1, fl_kind = kFlushPlain, fl_comp = 0, fl_stride = 1;
+  float fl_scale = 1.0f;
+  float* fl_base = v_opacities;
+  if (fc < CH) {
+    fl_word0 = fc, fl_base = v_colors, fl_stride = CH, fl_comp = fc;
+  } else if (fc < CH + 3) {
+    fl_word0 = fc, fl_base = v_conics, fl_stride = 3, fl_comp = fc - CH, fl_scale = fc - CH == 1 ? 1.0f : 0.5f;
+  } else if (fc < CH + 5) {
+    fl_word0 = CH + 3, fl_word1 = CH + 4, fl_kind = kFlushMean, fl_base = v_means2d, fl_stride = 2, fl_comp = fc - CH - 3;
+  } else if (fc == CH + 5) {
+    fl_word0 = CH + 5, fl_kind = kFlushOpacity, fl_base = v_opacities;
+  }
+
+  const int64_t unit = blockIdx.x;
+  if (unit >= n_units) return;  // uniform across the block
+  const int64_t it = order[unit];
+  const int64_t image = it / n_tiles;
+  const int tile = static_cast<int>(it % n_tiles);
+  const int tx = tile % a.tw, ty = tile / a.tw;
+  int64_t start, end;
+  tile_range(a, image, tile, &start, &end);
+  const int64_t stop = start + cost[it];
+  int32_t r_id = 0;
+  float2 r_xy = make_float2(0.0f, 0.0f);
+  float4 r_co = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  int32_t r_g = 0;
+  float r_col[CH];
+  auto load_ids = [&](int64_t hi, int64_t lo) {
+    const int64_t j = hi - 1 - t;
+    if (t < BB && j >= lo) r_id = a.flatten_ids[j];
+  };
+  auto load_records = [&](int64_t hi, int64_t lo) {  // of the ids in r_id
+    const int64_t j = hi - 1 - t;
+    if (t < BB && j >= lo) {
+      const int32_t g = r_id;
+      const bool ok = g >= 0 && static_cast<int64_t>(g) < a.G;
+      const int64_t gg = ok ? g : 0;
+      r_g = ok ? g : 0;
+      if (ok) {
+        r_xy = make_float2(a.means2d[gg * 2], a.means2d[gg * 2 + 1]);
+        r_co = make_float4(a.conics[gg * 3], a.conics[gg * 3 + 1], a.conics[gg * 3 + 2], a.opacities[gg]);
+      } else {
+        r_xy = make_float2(0.0f, 0.0f);
+        r_co = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+#pragma unroll
+      for (int c = 0; c < CH; ++c) r_col[c] = ok ? a.colors[gg * CH + c] : 0.0f;
+    }
+  };
+  if (stop > start) {
+    const int64_t lo0 = max<int64_t>(start, stop - BB);
+    load_ids(stop, lo0);
+    load_records(stop, lo0);
+  }
+
+  store_wave_rects(s_rect, n_waves, a.ts, tx, ty);
+  int wave_last;
+  bool wave_rc_finite;
+  {
+    int qx, qy;
+    lane_pixel(t, a.ts, &qx, &qy);
+    const int x = tx * a.ts + qx;
+    const int y = ty * a.ts + qy;
+    const bool inside = t < a.ts * a.ts && x < a.W && y < a.H;
+    const int64_t pix = (image * a.H + y) * static_cast<int64_t>(a.W) + x;
+    const float T_final = inside ? 1.0f - render_alphas[pix] : 1.0f;
+    int last_rel = -1;  // last contributor relative to start, -1 for none
+    if (inside) {
+      const int64_t l = min<int64_t>(end - 1, last_ids[pix]) - start;
+      last_rel = static_cast<int>(max<int64_t>(-1, min<int64_t>(l, INT32_MAX - 1)));
+    }
+    float v_rc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float bg_dot = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) v_rc[c] = inside ? v_render_colors[pix * CH + c] : 0.0f;
+    const float v_ra = inside && v_render_alphas ? v_render_alphas[pix] : 0.0f;
+    if (a.backgrounds) {
+      const float* bg = a.backgrounds + image * CH;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) bg_dot += bg[c] * v_rc[c];
+    }
+    const float coef = T_final * v_ra + -T_final * bg_dot;
+    bool rc_finite = fabsf(T_final) <= 3.402823466e38f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) rc_finite = rc_finite && fabsf(v_rc[c]) <= 3.402823466e38f;
+    wave_rc_finite = __ballot(!rc_finite) == 0;
+    wave_last = last_rel;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) wave_last = max(wave_last, __shfl_xor(wave_last, off, kWave));
+    s_pix[t] = make_float4(v_rc[0], v_rc[1], v_rc[2], CH == 4 ? v_rc[3] : __int_as_float(last_rel));
+    s_state[t] = make_float2(T_final, coef);
+    if constexpr (CH == 4) s_last[t] = last_rel;
+    if (t < kNeutral) s_neutral[t] = make_float2(1.0f, 0.0f);  // read after the batch loop's first barrier
+  }
+  const PixRect wr = wave_rect(wave, a.ts, tx, ty);
+  const int ri = lane & 15, rk = lane >> 4;  // record of the group, pixel row (and row + 4)
+  const float4* pix_row = s_pix + wave * kWave + rk * 8;
+  float2* state_row = s_state + wave * kWave + rk * 8;
+  // lane 0 of the row brings the pixel's state into the scans, the others
+  // their neutral elements
+  const float2* state_in = ri == 0 ? state_row : s_neutral;
+  const int* last_row = s_last + wave * kWave + rk * 8;  // CH == 4 only
+  uint16_t* list = s_list + wave * BB;
+  const float py0 = wr.y0 + static_cast<float>(rk), py1 = wr.y0 + static_cast<float>(rk + 4);
+
+  int skip = 0;  // slots of the batch that this wave has already evaluated
+  for (int64_t b1 = stop; b1 > start;) {
+    const int64_t b0 = max<int64_t>(start, b1 - BB);
+    __syncthreads();  // previous batch fully consumed and flushed
+    if (t < BB && b1 - 1 - t >= b0) {
+      const uint32_t cls = record_class(r_xy, r_co);
+      const uint32_t r_mask = touch_mask(r_xy, r_co, n_waves, s_rect) | cls;
+      float* rec = s_rec + t * RW;
+      *reinterpret_cast<float4*>(rec) = make_float4(0.5f * r_co.x, r_co.y, 0.5f * r_co.z, r_co.w);
+      float tail[RW - 4];
+#pragma unroll
+      for (int i = 0; i < RW - 4; ++i) tail[i] = 0.0f;
+      tail[0] = r_xy.x;
+      tail[1] = r_xy.y;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) tail[2 + c] = r_col[c];
+      tail[GW - 4] = __int_as_float(r_g);
+      bool rec_finite = fabsf(r_xy.x) <= 3.402823466e38f && fabsf(r_xy.y) <= 3.402823466e38f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) rec_finite = rec_finite && fabsf(r_col[c]) <= 3.402823466e38f;
+      tail[GW - 3] = __uint_as_float(r_mask | (rec_finite ? 0u : kNonFiniteRecord));
+#pragma unroll
+      for (int i = 0; i < RW - 4; i += 4)
+        *reinterpret_cast<float4*>(rec + 4 + i) = make_float4(tail[i], tail[i + 1], tail[i + 2], tail[i + 3]);
+    }
+    for (int w = t; w < BB * NS; w += BS) s_acc[w] = 0.0;
+    __syncthreads();
+    const int cnt = static_cast<int>(b1 - b0);
+    const int k_rel0 = static_cast<int>(b1 - 1 - start);  // entry of slot 0, relative to start
+    int n = 0;
+    for (int c0 = 0; c0 < cnt; c0 += kWave) {
+      const int kl = c0 + lane;
+      const uint32_t mk = kl < cnt ? s_mask(kl) : 0u;
+      const bool mine = kl >= skip && k_rel0 - kl <= wave_last && ((mk >> wave) & 1u);
+      const uint64_t bits = __ballot(mine);
+      const int below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bits >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bits), 0));
+      if (mine) list[n + below] = static_cast<uint16_t>(kl);
+      n += __popcll(bits);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // list: written and read by this wave
+    // Only whole groups are evaluated while entries remain before this batch:
+    // the next one starts at the first slot that some wave left over, unless
+    // that wave's few records reach back too far.
+    int left = cnt;  // this wave's first slot left over
+    if (b0 > start && (n & 15)) {
+      const int first = __builtin_amdgcn_readfirstlane(static_cast<int>(list[n & ~15]));
+      if (first >= kRowsAdvance) {
+        left = first;
+        n &= ~15;
+      }
+    }
+    if (lane == 0) s_next[wave] = left;
+    __syncthreads();
+    int advance = cnt;
+    for (int w = 0; w < n_waves; ++w) advance = min(advance, s_next[w]);
+    skip = left - advance;
+    const int64_t b1n = b1 - advance;
+    const int64_t b0n = max<int64_t>(start, b1n - BB);
+    // the next batch's ids, then (behind the first group) its records
+    load_ids(b1n, b0n);
+    if (n == 0) load_records(b1n, b0n);
+    for (int g0 = 0; g0 < n; g0 += 16) {
+      const bool live = g0 + ri < n;
+      const int slot = list[min(g0 + ri, n - 1)];
+      const float* rec = s_rec + slot * RW;
+      const float4 co = reinterpret_cast<const float4*>(rec)[0];
+      const float4 xc = reinterpret_cast<const float4*>(rec)[1];
+      float4 ex = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if constexpr (RW > 8) ex = reinterpret_cast<const float4*>(rec)[2];
+      const float col[4] = {xc.z, xc.w, ex.x, ex.y};
+      const uint32_t bits = s_mask(slot);
+      const int k_rel = live ? k_rel0 - slot : INT_MAX;
+      const float dy[2] = {xc.y - py0, xc.y - py1};
+      const float cy[2] = {co.z * dy[0] * dy[0], co.z * dy[1] * dy[1]};
+      float vc[CH], S[2] = {0.0f, 0.0f}, Hx[2] = {0.0f, 0.0f}, Hxx = 0.0f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) vc[c] = 0.0f;
+      auto walk = [&](auto level_c) {
+        constexpr int kLevel = decltype(level_c)::value;
+        constexpr bool kCareful = kLevel == 2;
+        float px = wr.x0;
+        const float4* pix = pix_row;
+        const float2* in = state_in;
+        float2* out = state_row;
+#pragma unroll 1
+        for (int x = 0; x < 8; x += 2, pix += 2, in += 2, out += 2) {
+          float4 vr[4];
+          float Tn[4], Bb[4], al[4], araw[4], ra[4], fac[4], D[4], Ba[4];
+          bool valid[4];
+          float dx[2];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {  // q = 2 * column + half
+            const int at = (q >> 1) + 32 * (q & 1);
+            vr[q] = pix[at];
+            const float2 st = in[at];
+            Tn[q] = st.x;
+            Bb[q] = st.y;
+            const int last = CH == 4 ? last_row[x + at] : __float_as_int(vr[q].w);
+            valid[q] = k_rel <= last;
+          }
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            dx[p] = xc.x - px;
+            px += 1.0f;
+            const float ax = co.x * dx[p] * dx[p];
+            const float bx = co.y * dx[p];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int q = 2 * p + h;
+              const float sigma = (ax + cy[h]) + bx * dy[h];  // halved_sigma's operations
+              float alpha;
+              if constexpr (kLevel < 2) {
+                araw[q] = co.w * exp_alpha_bounded(-sigma);
+                alpha = kLevel == 0 ? araw[q] : fminf(kMaxAlpha, araw[q]);
+                valid[q] = valid[q] && alpha >= kAlphaThreshold;
+              } else {
+                araw[q] = co.w * exp_alpha(-sigma);
+                alpha = fminf(kMaxAlpha, araw[q]);
+                valid[q] = valid[q] && !(sigma < 0.0f || alpha < kAlphaThreshold);
+              }
+              al[q] = valid[q] ? alpha : 0.0f;
+              ra[q] = __builtin_amdgcn_rcpf(1.0f - al[q]);  // alpha <= 0.99; 1 for alpha = 0
+              Tn[q] *= ra[q];
+            }
+          }
+          row16_product4(Tn);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            fac[q] = al[q] * Tn[q];
+            const float vrq[4] = {vr[q].x, vr[q].y, vr[q].z, vr[q].w};
+            D[q] = col[0] * vrq[0];
+#pragma unroll
+            for (int c = 1; c < CH; ++c) D[q] = __builtin_fmaf(col[c], vrq[c], D[q]);
+            if constexpr (kCareful) {
+              Ba[q] = valid[q] ? __builtin_fmaf(-fac[q], D[q], Bb[q]) : Bb[q];
+#pragma unroll
+              for (int c = 0; c < CH; ++c) vc[c] += valid[q] ? fac[q] * vrq[c] : 0.0f;
+            } else {
+              Ba[q] = __builtin_fmaf(-fac[q], D[q], Bb[q]);
+#pragma unroll
+              for (int c = 0; c < CH; ++c) vc[c] = __builtin_fmaf(fac[q], vrq[c], vc[c]);
+            }
+          }
+          row16_sum4(Ba, Bb);
+          if (ri == 15) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[(q >> 1) + 32 * (q & 1)] = make_float2(Tn[q], Ba[q]);
+          }
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            float vs[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int q = 2 * p + h;
+              const float v_alpha = __builtin_fmaf(Tn[q], D[q], ra[q] * Bb[q]);
+              vs[h] = -al[q] * v_alpha;
+              if constexpr (kLevel == 1) vs[h] = araw[q] <= kMaxAlpha ? vs[h] : 0.0f;
+              if constexpr (kLevel == 2) vs[h] = valid[q] && araw[q] <= kMaxAlpha ? vs[h] : 0.0f;
+              S[h] += vs[h];
+              Hx[h] = __builtin_fmaf(vs[h], dx[p], Hx[h]);
+            }
+            Hxx = __builtin_fmaf(vs[0] + vs[1], dx[p] * dx[p], Hxx);
+          }
+        }
+      };
+      int level = 0;
+      if (__ballot(live && (bits & kCappedRecord)) != 0) level = 1;
+      if (!wave_rc_finite || __ballot(live && (bits & (kGeneralRecord | kNonFiniteRecord))) != 0) level = 2;
+      if (level == 0) {
+        walk(std::integral_constant<int, 0>{});
+      } else if (level == 1) {
+        walk(std::integral_constant<int, 1>{});
+      } else {
+        walk(std::integral_constant<int, 2>{});
+      }
+      float v[NV];
+#pragma unroll
+      for (int c = 0; c < CH; ++c) v[c] = vc[c];
+      v[CH + 0] = Hxx;
+      v[CH + 1] = __builtin_fmaf(Hx[1], dy[1], Hx[0] * dy[0]);
+      const float sy0 = S[0] * dy[0], sy1 = S[1] * dy[1];
+      v[CH + 2] = __builtin_fmaf(sy1, dy[1], sy0 * dy[0]);
+      v[CH + 3] = Hx[0] + Hx[1];
+      v[CH + 4] = sy0 + sy1;
+      v[CH + 5] = S[0] + S[1];
+      if (level == 2 && (bits & kNonFiniteRecord) && !(fabsf(xc.x) <= 3.402823466e38f && fabsf(xc.y) <= 3.402823466e38f)) {
+        // no pixel has a geometry term under a non-finite mean
+#pragma unroll
+        for (int i = CH; i < NV; ++i) v[i] = 0.0f;
+      }
+      // sums over the four rows: after the two exchanges a lane with bits
+      // h = lane[5], r = lane[4] holds component 4 m + 2 r + h in y[m]
+      constexpr int NA = (NV + 1) / 2, NB = (NA + 1) / 2;
+      float w[NA], y[NB];
+      unsigned spare = 0u;
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const unsigned b = (2 * i + 1 < NV) ? ubits(v[2 * i + 1]) : spare;
+        const auto sw = __builtin_amdgcn_permlane32_swap(ubits(v[2 * i]), b, false, false);
+        w[i] = fbits(sw[0]) + fbits(sw[1]);
+        spare = sw[1];
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const unsigned b = (2 * i + 1 < NA) ? ubits(w[2 * i + 1]) : spare;
+        const auto sw = __builtin_amdgcn_permlane16_swap(ubits(w[2 * i]), b, false, false);
+        y[i] = fbits(sw[0]) + fbits(sw[1]);
+        spare = sw[1];
+      }
+      if (live) {
+        const int comp0 = 2 * (rk & 1) + (rk >> 1);
+        double* acc = s_acc + slot * NS + comp0;
+#pragma unroll
+        for (int m = 0; m < NB; ++m) {
+          const int c = 4 * m + comp0;
+          if (4 * m + 3 < NV || c < NV)
+            __hip_atomic_fetch_add(acc + 4 * m, static_cast<double>(y[m]), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      }
+      if (g0 == 0) load_records(b1n, b0n);
+    }
+    __syncthreads();
+    __builtin_amdgcn_s_waitcnt(kWaitVmemOnly);
+    for (int idx = t; idx < cnt * kFlushLanes; idx += BS) {
+      const int slot = idx / kFlushLanes;
+      if (fl_word0 < 0) continue;  // lanes past the slot's components
+      float v = static_cast<float>(s_acc[slot * NS + fl_word0]);
+      const int64_t gg = s_g(slot);
+      if (fl_kind == kFlushMean) {
+        const float v2 = static_cast<float>(s_acc[slot * NS + fl_word1]);
+        if (v == 0.0f && v2 == 0.0f) continue;
+        const float4 co = *reinterpret_cast<const float4*>(s_rec + slot * RW);
+        v = fl_comp == 0 ? (co.x + co.x) * v + co.y * v2 : co.y * v + (co.z + co.z) * v2;
+      } else if (fl_kind == kFlushOpacity) {
+        if (v == 0.0f) continue;
+        v = -v / s_rec[slot * RW + 3];
+      } else {
+        v *= fl_scale;
+      }
+      if (v != 0.0f) unsafeAtomicAdd(fl_base + gg * fl_stride + fl_comp, v);
+    }
+    b1 = b1n;
+  }
+}
+
 // Heavy-first tile schedule for the backward. A tile's cost is the number of
 // list entries its pixels replay (largest last_id - start + 1, 0 when masked
 // or empty). The backward launches one block per tile in descending cost
@@ -1250,6 +1744,17 @@ size_t bwd_smem(int ch, int bs, int bb, bool absgrad) {
   return static_cast<size_t>(bb) * (bwd_record_words(ch) + (bs / kWave) * ns) * 4 + static_cast<size_t>(bs / kWave) * 16;
 }
 
+// The rows kernel: accumulators, pixel cotangents and state, records, wave
+// rectangles and record lists, in the kernel's order.
+int bwd_rows_batch(int bs) { return std::min(bs, kRowsBatch); }
+size_t bwd_rows_smem(int ch, int bs, int bb) {
+  const size_t ns = static_cast<size_t>(ch + 6) | 1;
+  const size_t acc = (static_cast<size_t>(bb) * ns + 1) / 2 * 16;
+  const size_t words = static_cast<size_t>(bs) * (ch == 4 ? 7 : 6) + 2 * kNeutral +
+                       static_cast<size_t>(bb) * bwd_record_words(ch) + 5 * (bs / kWave);
+  return acc + words * 4 + static_cast<size_t>(bs / kWave) * bb * 2;
+}
+
 int check_args(const RasterArgs& a, const char* what) {
   if (a.I < 0 || a.N < 0 || a.channels <= 0 || a.W < 0 || a.H < 0 || a.ts <= 0 || a.tw < 0 || a.th < 0 ||
       a.n_isects < 0)
@@ -1544,13 +2049,35 @@ static int rasterize_bwd_impl(const float* means2d, const float* conics, const f
                                                           v_backgrounds);
   }
   if ((rc = check_launch("rasterize_to_pixels_3dgs_backward"))) return rc;
+  KernelTimer timer("raster_bwd", s);
+  const unsigned nb = static_cast<unsigned>(n_total);
+  // one block per tile (block b: the tile of rank b in the heavy-first order)
+  //
+  // Records in lanes wherever that kernel applies: whole 8x8 pixel blocks,
+  // staged colours, sums of signed gradients only, pixel centres exact in
+  // float under + 1 steps.
+  constexpr int kExactCentres = 1 << 22;
+  if (ch >= 1 && !v_means2d_abs && tile_size % 8 == 0 && image_width <= kExactCentres &&
+      image_height <= kExactCentres) {
+    const int bb = bwd_rows_batch(bs);
+    const size_t sm = bwd_rows_smem(ch, bs, bb);
+#define GSPLAT_BWD_ROWS(C)                                                                                     \
+  raster_bwd_rows_kernel<C><<<nb, bs, sm, s>>>(a, bb, n_total, order, cost, render_alphas, last_ids,           \
+                                               v_render_colors, v_render_alphas, v_means2d, v_conics, v_colors, \
+                                               v_opacities)
+    switch (ch) {
+      case 1: GSPLAT_BWD_ROWS(1); break;
+      case 2: GSPLAT_BWD_ROWS(2); break;
+      case 3: GSPLAT_BWD_ROWS(3); break;
+      default: GSPLAT_BWD_ROWS(4); break;
+    }
+#undef GSPLAT_BWD_ROWS
+    return check_launch("rasterize_to_pixels_3dgs_backward");
+  }
   const int bb = bwd_batch(bs);
   const size_t sm = bwd_smem(ch, bs, bb, v_means2d_abs != nullptr);
-  KernelTimer timer("raster_bwd", s);
-  // one block per tile (block b: the tile of rank b in the heavy-first order)
 #define GSPLAT_BWD_LAUNCH(C, ABS_, VABS)                                                                       \
   {                                                                                                            \
-    const unsigned nb = static_cast<unsigned>(n_total);                                                        \
     raster_bwd_kernel<C, ABS_><<<nb, bs, sm, s>>>(a, bb, n_total, order, cost, render_alphas, last_ids,       \
                                                   v_render_colors, v_render_alphas, VABS, v_means2d, v_conics, \
                                                   v_colors, v_opacities, v_backgrounds);                        \

@@ -1,0 +1,82 @@
+"""The rasterize backward with records in lanes (tile sides that are multiples
+of 8, one to four channels, no absolute gradients) against the oracle, where
+its groups of 16 records, its batches of 256 entries and its record classes
+meet: list lengths around 16 and 256, every tile side it takes, opacities over
+the 0.99 cap, ill-conditioned conics, opacities over 1 and non-finite records.
+
+Tolerance: the gradients' usual bar, 1e-3 of each element or of 1% of the
+tensor's largest (both sides round every pixel's terms in float32; the sums
+run in another order).
+"""
+import numpy as np
+import pytest
+
+from _helpers import assert_close_rel, dev, gsplat, host
+from test_gpu_raster import GRAD_RTOL, _oracle_fwd, _raster_inputs, make_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(oracle, s, W, H, ts, rng, finite=True):
+    g = gsplat()
+    got = g.rasterize_to_pixels_3dgs_forward(_raster_inputs(s), W, H, ts)
+    exp = _oracle_fwd(oracle, s, W, H, ts)
+    np.testing.assert_array_equal(host(got["last_ids"]), exp["last_ids"])
+    v_rc = rng.normal(size=exp["render_colors"].shape).astype(np.float32)
+    v_ra = rng.normal(size=exp["render_alphas"].shape).astype(np.float32)
+    bwd = g.rasterize_to_pixels_3dgs_backward(
+        _raster_inputs(s), {"render_alphas": got["render_alphas"], "last_ids": got["last_ids"]},
+        {"v_render_colors": dev(v_rc), "v_render_alphas": dev(v_ra)}, W, H, ts)
+    want = oracle.raster_backward(s["means2d"], s["conics"], s["colors"], s["opacities"], s["tile_offsets"],
+                                  s["flatten_ids"], W, H, ts, exp["render_alphas"], exp["last_ids"], v_rc, v_ra,
+                                  backgrounds=s["backgrounds"], masks=s.get("masks"))
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        a, e = host(bwd[k]), want[k]
+        if not finite:
+            np.testing.assert_array_equal(np.isfinite(a), np.isfinite(e), err_msg=k)
+            a, e = np.where(np.isfinite(e), a, 0), np.where(np.isfinite(e), e, 0)
+        assert_close_rel(a, e, GRAD_RTOL, k)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 255, 256, 257, 529])
+def test_list_lengths(oracle, n):
+    """One tile whose list holds about n faint records (every group and batch remainder)."""
+    rng = np.random.default_rng(n)
+    s = make_scene(oracle, rng, 1, n, 16, 16, 16, 3, opac=(0.006, 0.03), scale=(4.0, 9.0))
+    _check(oracle, s, 16, 16, 16, rng)
+
+
+@pytest.mark.parametrize("ts,C,W,H,masks", [(8, 3, 61, 45, False), (16, 1, 50, 33, True), (16, 2, 70, 40, False),
+                                            (24, 4, 75, 50, False), (32, 3, 97, 64, True), (16, 4, 33, 47, False)])
+def test_tile_sides_and_channels(oracle, ts, C, W, H, masks):
+    rng = np.random.default_rng(ts + C)
+    s = make_scene(oracle, rng, 2, 900, W, H, ts, C, opac=(0.05, 0.9), masks=masks)
+    _check(oracle, s, W, H, ts, rng)
+
+
+@pytest.mark.parametrize("opac", [(0.9, 0.99), (0.97, 1.0), (1.0, 1.7)])
+def test_capped_and_general_opacities(oracle, opac):
+    """Groups with records over the cap and over 1 beside plain ones."""
+    rng = np.random.default_rng(7)
+    s = make_scene(oracle, rng, 1, 600, 48, 48, 16, 3, opac=(0.05, 0.6), scale=(1.0, 3.0))
+    pick = rng.random(s["opacities"].shape) < 0.2
+    s["opacities"] = np.where(pick, rng.uniform(*opac, s["opacities"].shape), s["opacities"]).astype(np.float32)
+    _check(oracle, s, 48, 48, 16, rng)
+
+
+def test_ill_conditioned_and_non_finite_records(oracle):
+    """Records of the general class in groups of plain ones: conics close to
+    singular, not positive definite and huge, infinite and NaN means and colours."""
+    rng = np.random.default_rng(11)
+    W = H = 48
+    s = make_scene(oracle, rng, 1, 500, W, H, 16, 3, opac=(0.05, 0.6), scale=(1.0, 4.0))
+    con = s["conics"].reshape(-1, 3)
+    con[3] = [0.2, 0.199999, 0.2]
+    con[40] = [0.2, 0.3, 0.2]
+    con[77] = [3.0e7, 0.0, 2.0e7]
+    con[120] = [1.0e-18, 0.0, 0.3]
+    mean = s["means2d"].reshape(-1, 2)
+    mean[200] = [np.inf, 20.0]
+    s["colors"].reshape(-1, 3)[250, 1] = np.inf
+    s["colors"].reshape(-1, 3)[300, 2] = np.nan
+    _check(oracle, s, W, H, 16, rng, finite=False)
