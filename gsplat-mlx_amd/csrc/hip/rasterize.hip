@@ -50,6 +50,9 @@ constexpr int kMaxChannels = 64;
 // per-wave touch mask, padded to 16 bytes.
 __host__ __device__ constexpr int bwd_record_words(int ch) { return 4 + (2 + ch + 2 + 3) / 4 * 4; }
 
+// The rows kernels' forward record also carries the touch mask.
+__host__ __device__ constexpr int fwd_rows_record_words(int ch) { return 4 + (2 + ch + 1 + 3) / 4 * 4; }
+
 struct RasterArgs {
   const float* means2d;
   const float* conics;
@@ -472,6 +475,287 @@ __global__ void __launch_bounds__(1024) raster_fwd_kernel(RasterArgs a, float* _
   } else {
     for (int c = 0; c < channels; ++c) render_colors[pix * channels + c] = acc[c] + T * (bg ? bg[c] : 0.0f);
   }
+  last_ids[pix] = cur;
+}
+
+// The pixels of a wave and of its lanes in the kernels that keep 16 records in
+// lanes: lane l holds record l % 16 of a group and, in lane group l / 16, NX
+// columns of two rows of the wave's BX x BY pixel block. P = 64: an 8x8 block,
+// lane group g has rows g and g + 4. P = 32 (8x4) and P = 16 (4x4): lane groups
+// are 2 x 2 over the block, two adjacent rows each. Pixel (x, y) of the block
+// has index y BX + x.
+template <int P>
+struct RowBlock {
+  static constexpr int BX = P == 16 ? 4 : 8, BY = P / BX;
+  static constexpr int NX = P / 8;                    // columns of a lane
+  static constexpr int HS = P == 64 ? 4 : 1;          // rows between a lane's two
+  static __device__ __forceinline__ int x0(int g) { return P == 64 ? 0 : (g & 1) * NX; }
+  static __device__ __forceinline__ int y0(int g) { return P == 64 ? g : (g >> 1) * 2; }
+  static __host__ __device__ constexpr int waves(int ts) { return ts * ts / P; }
+  static __device__ __forceinline__ PixRect rect(int w, int ts, int tx, int ty) {
+    const int bpr = ts / BX;
+    PixRect r;
+    r.x0 = static_cast<float>(tx * ts + (w % bpr) * BX) + 0.5f;
+    r.x1 = r.x0 + static_cast<float>(BX - 1);
+    r.y0 = static_cast<float>(ty * ts + (w / bpr) * BY) + 0.5f;
+    r.y1 = r.y0 + static_cast<float>(BY - 1);
+    return r;
+  }
+};
+
+// Forward with records in lanes: tile sides 8, 16 and 24, one to four channels.
+// Staging and culling are raster_fwd_kernel's, and so are every alpha,
+// transmittance and sum, bit for bit. A wave takes the records that may touch
+// its pixels in groups of 16, in two steps:
+// 1. records in lanes: each lane evaluates the alphas of its record at its
+//    columns and rows (RowBlock; a column's (0.5 c0 dx) dx and c1 dx serve two
+//    rows, a row's (0.5 c2 dy) dy every column) and stores them in LDS, 0 where
+//    the alpha test fails. Groups without capped or general records skip the
+//    cap's and sigma's tests.
+// 2. one pixel per lane: the group's records in list order, without a branch.
+//
+// The kernel with pixels in lanes throughout was bound by VALU issue too (0.99):
+// 37 instructions per (wave, record) visit and 22 scalar ones for the visits'
+// bit masks and branches, here 17 + 11 and few: 155 -> 135 us at 1M Gaussians,
+// 1297x840 (1.81 -> 1.73 ms over 8 images of 1920x1080, 714 -> 671 us at
+// 3840x2160). Batches of 128 records keep 6 blocks per CU by LDS (135 us, 192:
+// 142 us, 256: 161 us). Skipping step 2's tests in waves whose pixels all
+// stay live was slower (138 us), as was branching around records.
+//
+// Small grids (P < 64, the tile split over 64 / P blocks of its own): few tiles
+// leave most SIMDs idle while the heaviest tile runs, so a tile's 8x8 pixel
+// blocks are cut into 8x4 or 4x4 ones with a wave each, and a block takes half
+// or a quarter of the tile. More waves repeat step 2's lanes and the staging,
+// so this stops paying once the tiles fill the chip (10,000 Gaussians at
+// 256x256, 256 tiles: 61 us before, 40 at P = 64, 31 at 32, 29 at 16; at
+// 320x320 106, 87 and 98 us for 700,000 Gaussians; from 1024 tiles on P = 64
+// is the fastest).
+constexpr int kRowsBatch = 256;
+constexpr int kRowsSmallBatch = 128;
+
+template <int CH, int P>
+__global__ void __launch_bounds__(576) raster_fwd_rows_kernel(RasterArgs a, int BB, int split,
+                                                               float* __restrict__ render_colors,
+                                                               float* __restrict__ render_alphas,
+                                                               int32_t* __restrict__ last_ids) {
+  using RB = RowBlock<P>;
+  constexpr int FW = fwd_rows_record_words(CH);
+  constexpr int MW = 6 + CH;  // word of the touch mask and class
+  constexpr int PS = P + 4;  // alpha words per record: 16 records' rows start in distinct banks
+  extern __shared__ float smem[];
+  const int BS = blockDim.x;
+  const int n_waves = BS / kWave;
+  float* s_rec = smem;                                                    // [BB][FW]
+  float* s_alpha = s_rec + BB * FW;                                       // [n_waves][16][PS]
+  float4* s_col = reinterpret_cast<float4*>(s_alpha + n_waves * 16 * PS);  // [n_waves][16] colours (and entry)
+  float4* s_rect = s_col + n_waves * 16;                                  // [n_waves]
+  int* s_pos = reinterpret_cast<int*>(s_rect + n_waves);                  // [n_waves][16] entry (CH == 4)
+  uint8_t* s_list = reinterpret_cast<uint8_t*>(s_pos + (CH == 4 ? n_waves * 16 : 0));  // [n_waves][BB]
+  auto s_mask = [&](int k) { return __float_as_uint(s_rec[k * FW + MW]); };
+
+  const int tx = blockIdx.x / split, ty = blockIdx.y;
+  const int64_t image = blockIdx.z;
+  const int tile = ty * a.tw + tx;
+  const int t = threadIdx.x;
+  const int lane = t % kWave;
+  const int wave = t / kWave;
+  const int wave0 = (blockIdx.x % split) * n_waves;  // this block's first wave of the tile
+  const int bpr = a.ts / RB::BX;
+  const int x = tx * a.ts + ((wave0 + wave) % bpr) * RB::BX + lane % RB::BX;
+  const int y = ty * a.ts + ((wave0 + wave) / bpr) * RB::BY + (lane % P) / RB::BX;
+  const bool inside = lane < P && x < a.W && y < a.H;
+  const int64_t pix = (image * a.H + y) * static_cast<int64_t>(a.W) + x;
+  const float* bg = a.backgrounds ? a.backgrounds + image * CH : nullptr;
+  const int64_t n_tiles = static_cast<int64_t>(a.tw) * a.th;
+
+  if (a.masks && !a.masks[image * n_tiles + tile]) {
+    if (inside) {
+      render_alphas[pix] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) render_colors[pix * CH + c] = bg ? bg[c] : 0.0f;
+      last_ids[pix] = 0;
+    }
+    return;
+  }
+  int64_t start, end;
+  tile_range(a, image, tile, &start, &end);
+  if (t < n_waves) {
+    const PixRect r = RB::rect(wave0 + t, a.ts, tx, ty);
+    s_rect[t] = make_float4(r.x0, r.x1, r.y0, r.y1);
+  }
+  const PixRect wr = RB::rect(wave0 + wave, a.ts, tx, ty);
+  const int ri = lane & 15, rk = lane >> 4;
+  const float lx0 = wr.x0 + static_cast<float>(RB::x0(rk));
+  const float py0 = wr.y0 + static_cast<float>(RB::y0(rk)), py1 = py0 + static_cast<float>(RB::HS);
+  float* alpha_out = s_alpha + (wave * 16 + ri) * PS + RB::y0(rk) * RB::BX + RB::x0(rk);
+  const float* alpha_in = s_alpha + wave * 16 * PS + lane % P;
+  float4* wave_col = s_col + wave * 16;
+  int* wave_pos = s_pos + wave * 16;
+  uint8_t* list = s_list + wave * BB;
+
+  // T > 0: the pixel's transmittance; T < 0: minus the final one (saturated,
+  // or no pixel)
+  float T = inside ? 1.0f : -1.0f;
+  int32_t cur = 0;
+  float acc[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) acc[c] = 0.0f;
+
+  float2 r_xy = make_float2(0.0f, 0.0f);
+  float4 r_co = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float r_col[CH];
+  auto load_records = [&](int64_t b0) {
+    const int64_t j = b0 + t;
+    if (t < BB && j < end) {
+      const int32_t g = load_gaussian(a, j, &r_xy, &r_co);
+#pragma unroll
+      for (int c = 0; c < CH; ++c) r_col[c] = a.colors[static_cast<int64_t>(g) * CH + c];
+    }
+  };
+  load_records(start);
+  for (int64_t b0 = start; b0 < end; b0 += BB) {
+    if (__syncthreads_count(T < 0.0f) == BS) break;  // also fences the previous batch's LDS reads
+    if (t < BB && b0 + t < end) {
+      float* rec = s_rec + t * FW;
+      *reinterpret_cast<float4*>(rec) = make_float4(0.5f * r_co.x, r_co.y, 0.5f * r_co.z, r_co.w);
+      float tail[FW - 4];
+#pragma unroll
+      for (int i = 0; i < FW - 4; ++i) tail[i] = 0.0f;
+      tail[0] = r_xy.x;
+      tail[1] = r_xy.y;
+      bool finite = true;
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        tail[2 + c] = r_col[c];
+        finite = finite && fabsf(r_col[c]) <= 3.402823466e38f;
+      }
+      tail[MW - 4] = __uint_as_float(touch_mask(r_xy, r_co, n_waves, s_rect) | record_class(r_xy, r_co) |
+                                     (finite ? 0u : kNonFiniteRecord));
+#pragma unroll
+      for (int i = 0; i < FW - 4; i += 4)
+        *reinterpret_cast<float4*>(rec + 4 + i) = make_float4(tail[i], tail[i + 1], tail[i + 2], tail[i + 3]);
+    }
+    __syncthreads();
+    load_records(b0 + BB);
+    const int cnt = static_cast<int>(min<int64_t>(BB, end - b0));
+    int n = 0;
+    if (__ballot(T > 0.0f) != 0) {
+      for (int c0 = 0; c0 < cnt; c0 += kWave) {
+        const int kl = c0 + lane;
+        const bool mine = kl < cnt && ((s_mask(kl) >> wave) & 1u);
+        const uint64_t bits = __ballot(mine);
+        const int below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bits >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bits), 0));
+        if (mine) list[n + below] = static_cast<uint8_t>(kl);
+        n += __popcll(bits);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int g0 = 0; g0 < n; g0 += 16) {
+      const bool live = g0 + ri < n;
+      const int slot = list[min(g0 + ri, n - 1)];
+      const float* rec = s_rec + slot * FW;
+      float4 co = reinterpret_cast<const float4*>(rec)[0];
+      if (!live) co.w = 0.0f;  // alpha 0 past the list
+      const float4 xc = reinterpret_cast<const float4*>(rec)[1];
+      float4 ex = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if constexpr (FW > 8) ex = reinterpret_cast<const float4*>(rec)[2];
+      const uint32_t bits = s_mask(slot);
+      const int entry = static_cast<int>(b0) + slot;
+      if (rk == 0) {
+        wave_col[ri] = make_float4(xc.z, xc.w, ex.x, CH == 4 ? ex.y : __int_as_float(entry));
+        if constexpr (CH == 4) wave_pos[ri] = entry;
+      }
+      const float dy[2] = {xc.y - py0, xc.y - py1};
+      const float cy[2] = {co.z * dy[0] * dy[0], co.z * dy[1] * dy[1]};
+      auto falloffs = [&](auto level_c) {
+        constexpr int kLevel = decltype(level_c)::value;
+        float px = lx0;
+#pragma unroll
+        for (int cx = 0; cx < RB::NX; cx += 2) {
+          float al[2][2];
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const float dx = xc.x - px;
+            px += 1.0f;
+            const float ax = co.x * dx * dx;
+            const float bx = co.y * dx;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const float sigma = (ax + cy[h]) + bx * dy[h];  // halved_sigma's operations
+              float alpha;
+              bool pass;
+              if constexpr (kLevel < 2) {
+                alpha = co.w * exp_alpha_bounded(-sigma);
+                if constexpr (kLevel == 1) alpha = fminf(kMaxAlpha, alpha);
+                pass = alpha >= kAlphaThreshold;
+              } else {
+                alpha = fminf(kMaxAlpha, co.w * exp_alpha(-sigma));
+                pass = live && !(sigma < 0.0f || alpha < kAlphaThreshold);
+              }
+              al[h][p] = pass ? alpha : 0.0f;
+            }
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            *reinterpret_cast<float2*>(alpha_out + cx + h * RB::HS * RB::BX) = make_float2(al[h][0], al[h][1]);
+        }
+      };
+      if (__ballot(live && (bits & kCappedRecord)) == 0) {
+        falloffs(std::integral_constant<int, 0>{});
+      } else if (__ballot(live && (bits & kGeneralRecord)) == 0) {
+        falloffs(std::integral_constant<int, 1>{});
+      } else {
+        falloffs(std::integral_constant<int, 2>{});
+      }
+      const bool finite = __ballot(live && (bits & kNonFiniteRecord)) == 0;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // alphas and colours: written and read by this wave
+      // The group's records in list order, one pixel per lane, four at a time.
+      // The transmittance chain is one product per record: it never rises, so
+      // each record's test against the threshold stands alone.
+      auto composite4 = [&](int k0, auto careful_c) {
+        constexpr bool kCareful = decltype(careful_c)::value;
+        float al[4], tb[4], ta = T;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          al[k] = alpha_in[(k0 + k) * PS];
+          tb[k] = ta;
+          ta *= 1.0f - al[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float4 col = wave_col[k0 + k];
+          const float next_T = k < 3 ? tb[k < 3 ? k + 1 : 3] : ta;
+          const bool keep = next_T > kTransmittanceThreshold;
+          const float vis = keep ? al[k] * tb[k] : 0.0f;
+          T = keep ? next_T : -fabsf(T);
+          const bool take = vis > 0.0f;
+          const float cc[4] = {col.x, col.y, col.z, col.w};
+#pragma unroll
+          for (int c = 0; c < CH; ++c) {
+            const float v = __builtin_fmaf(cc[c], vis, acc[c]);
+            acc[c] = !kCareful || take ? v : acc[c];
+          }
+          cur = take ? (CH == 4 ? wave_pos[k0 + k] : __float_as_int(col.w)) : cur;
+        }
+      };
+      const int m = min(16, n - g0);
+      if (finite) {
+#pragma unroll
+        for (int k = 0; k < 16; k += 4)
+          if (k < m) composite4(k, std::false_type{});
+      } else {
+        for (int k = 0; k < m; k += 4) composite4(k, std::true_type{});
+      }
+      if (__ballot(T > 0.0f) == 0) break;  // every pixel of the wave has saturated
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  if (!inside) return;
+  T = fabsf(T);
+  render_alphas[pix] = 1.0f - T;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) render_colors[pix * CH + c] = acc[c] + T * (bg ? bg[c] : 0.0f);
   last_ids[pix] = cur;
 }
 
@@ -1004,8 +1288,7 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 }
 #undef GSPLAT_ROW_STEP
 
-// Backward with records in lanes: tiles whose side is a multiple of 8, one to
-// four channels, no absolute gradients (the training path). Block, schedule,
+// Backward with records in lanes: tile sides 8, 16 and 24, one to four channels, no absolute gradients (the training path). Block, schedule,
 // staging and flush are raster_bwd_kernel's; a wave still owns an 8x8 block of
 // pixels, but evaluates 16 records at a time: lane l holds record l % 16 of
 // the group (in list order, back to front) and the pixel rows l / 16 and
@@ -1027,7 +1310,8 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 //
 // - While entries remain before a batch, a wave evaluates whole groups only;
 //   the next batch starts at the first entry some wave left over (each wave
-//   skips what it has done). Groups then hold the same records whatever the
+//   skips what it has done, and the entries' sums move along, so an entry is
+//   flushed once). Groups then hold the same records whatever the
 //   tile's list holds beside them, so the same pixels' recurrences round the
 //   same with AABB and ellipse lists.
 //
@@ -1038,14 +1322,10 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 // 114 -> 81 us at 512x512. About 120 VGPRs hold four evaluations in flight
 // (their scans interleave without wait states); at five waves per SIMD (96
 // VGPRs) the loop spills, 293 us, and unrolled further it does at four.
-// Batches of 256 entries (4 blocks per CU by LDS) measured 231 us, 192 243 us
-// and 128 246 us (without the carried-over groups).
-constexpr int kRowsBatch = 256;
-constexpr int kRowsAdvance = 128;  // a batch advances by at least this many entries
 constexpr int kNeutral = 40;  // entries of the neutral state: columns 0-7 of two rows 32 apart
 
 template <int CH>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) raster_bwd_rows_kernel(
+__global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) raster_bwd_rows_kernel(
     RasterArgs a, int BB, int64_t n_units, const int32_t* __restrict__ order, const int32_t* __restrict__ cost,
     const float* __restrict__ render_alphas, const int32_t* __restrict__ last_ids,
     const float* __restrict__ v_render_colors, const float* __restrict__ v_render_alphas,
@@ -1182,6 +1462,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
   const float py0 = wr.y0 + static_cast<float>(rk), py1 = wr.y0 + static_cast<float>(rk + 4);
 
   int skip = 0;  // slots of the batch that this wave has already evaluated
+  int carried = 0, carried_from = 0;  // slots carried over, and the first of them in the last batch
   for (int64_t b1 = stop; b1 > start;) {
     const int64_t b0 = max<int64_t>(start, b1 - BB);
     __syncthreads();  // previous batch fully consumed and flushed
@@ -1206,7 +1487,16 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
       for (int i = 0; i < RW - 4; i += 4)
         *reinterpret_cast<float4*>(rec + 4 + i) = make_float4(tail[i], tail[i + 1], tail[i + 2], tail[i + 3]);
     }
-    for (int w = t; w < BB * NS; w += BS) s_acc[w] = 0.0;
+    // the sums of slots carried over move to the batch's first slots (at most
+    // half a batch, below the first one carried), the others clear
+    for (int w = t; w < BB * NS; w += BS) {
+      if (w < carried * NS) {
+        s_acc[w] = s_acc[carried_from * NS + w];
+        s_acc[carried_from * NS + w] = 0.0;
+      } else if (w < carried_from * NS || w >= (carried_from + carried) * NS) {
+        s_acc[w] = 0.0;
+      }
+    }
     __syncthreads();
     const int cnt = static_cast<int>(b1 - b0);
     const int k_rel0 = static_cast<int>(b1 - 1 - start);  // entry of slot 0, relative to start
@@ -1224,11 +1514,11 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // list: written and read by this wave
     // Only whole groups are evaluated while entries remain before this batch:
     // the next one starts at the first slot that some wave left over, unless
-    // that wave's few records reach back too far.
+    // that wave's few records reach back over half a batch.
     int left = cnt;  // this wave's first slot left over
     if (b0 > start && (n & 15)) {
       const int first = __builtin_amdgcn_readfirstlane(static_cast<int>(list[n & ~15]));
-      if (first >= kRowsAdvance) {
+      if (2 * first >= BB) {
         left = first;
         n &= ~15;
       }
@@ -1238,6 +1528,8 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     int advance = cnt;
     for (int w = 0; w < n_waves; ++w) advance = min(advance, s_next[w]);
     skip = left - advance;
+    carried = cnt - advance;
+    carried_from = advance;
     const int64_t b1n = b1 - advance;
     const int64_t b0n = max<int64_t>(start, b1n - BB);
     // the next batch's ids, then (behind the first group) its records
@@ -1406,7 +1698,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     }
     __syncthreads();
     __builtin_amdgcn_s_waitcnt(kWaitVmemOnly);
-    for (int idx = t; idx < cnt * kFlushLanes; idx += BS) {
+    for (int idx = t; idx < advance * kFlushLanes; idx += BS) {
       const int slot = idx / kFlushLanes;
       if (fl_word0 < 0) continue;  // lanes past the slot's components
       float v = static_cast<float>(s_acc[slot * NS + fl_word0]);
@@ -1744,9 +2036,28 @@ size_t bwd_smem(int ch, int bs, int bb, bool absgrad) {
   return static_cast<size_t>(bb) * (bwd_record_words(ch) + (bs / kWave) * ns) * 4 + static_cast<size_t>(bs / kWave) * 16;
 }
 
-// The rows kernel: accumulators, pixel cotangents and state, records, wave
+// The kernels with records in lanes take tiles of whole 8x8 pixel blocks whose
+// LDS stays below 64 KiB, in images whose pixel centres are exact floats under
+// + 1 steps.
+bool rows_kernels_apply(int ts, int width, int height) {
+  return (ts == 8 || ts == 16 || ts == 24) && width <= (1 << 22) && height <= (1 << 22);
+}
+
+// raster_fwd_rows_kernel: records, alphas, colours, wave rectangles, entries and
+// record lists.
+size_t fwd_rows_smem(int ch, int n_waves, int pixels, int bb) {
+  const size_t words = static_cast<size_t>(bb) * fwd_rows_record_words(ch) +
+                       static_cast<size_t>(n_waves) * (16 * (pixels + 4) + 64 + 4 + (ch == 4 ? 16 : 0));
+  return words * 4 + static_cast<size_t>(n_waves) * bb;
+}
+
+// raster_bwd_rows_kernel: accumulators, pixel cotangents and state, records, wave
 // rectangles and record lists, in the kernel's order.
-int bwd_rows_batch(int bs) { return std::min(bs, kRowsBatch); }
+// Batches: 256 entries leave the fewest barriers and flushes (1M Gaussians,
+// 4346 tiles: 232 us against 242 at 128); where all tiles are resident at once
+// (4 blocks on each of 256 CUs), 128 shorten the heaviest tiles' start (100,000
+// Gaussians, 1024 tiles: 79.6 us against 82.2).
+int bwd_rows_batch(int bs, int64_t n_tiles) { return std::min(bs, n_tiles <= 1024 ? kRowsSmallBatch : kRowsBatch); }
 size_t bwd_rows_smem(int ch, int bs, int bb) {
   const size_t ns = static_cast<size_t>(ch + 6) | 1;
   const size_t acc = (static_cast<size_t>(bb) * ns + 1) / 2 * 16;
@@ -1969,6 +2280,37 @@ static int rasterize_fwd_impl(const float* means2d, const float* conics, const f
   const int ch = channels <= 4 ? channels : 0;
   const size_t sm = fwd_smem(ch, bs);
   KernelTimer timer("raster_fwd", s);
+  // records in lanes wherever that kernel applies (pixel centres exact in
+  // float under + 1 steps), with smaller pixel blocks on small grids
+  const int64_t n_total = I * tile_width * static_cast<int64_t>(tile_height);
+  if (ch >= 1 && rows_kernels_apply(tile_size, image_width, image_height)) {
+    const int pixels = tile_size != 16 || n_total > 800 ? 64 : (n_total > 320 ? 32 : 16);
+    const int split = 64 / pixels;
+    const int n_waves = tile_size * tile_size / 64;
+    const int bb = std::min(n_waves * kWave, pixels == 64 ? kRowsSmallBatch : kRowsBatch);
+    const size_t rsm = fwd_rows_smem(ch, n_waves, pixels, bb);
+    const dim3 rgrid(static_cast<unsigned>(tile_width) * split, tile_height, static_cast<unsigned>(I));
+#define GSPLAT_FWD_ROWS(C, P)                                                                             \
+  raster_fwd_rows_kernel<C, P><<<rgrid, n_waves * kWave, rsm, s>>>(a, bb, split, render_colors, render_alphas, \
+                                                                   last_ids)
+#define GSPLAT_FWD_ROWS_P(C)      \
+  if (pixels == 64) {             \
+    GSPLAT_FWD_ROWS(C, 64);       \
+  } else if (pixels == 32) {      \
+    GSPLAT_FWD_ROWS(C, 32);       \
+  } else {                        \
+    GSPLAT_FWD_ROWS(C, 16);       \
+  }
+    switch (ch) {
+      case 1: GSPLAT_FWD_ROWS_P(1); break;
+      case 2: GSPLAT_FWD_ROWS_P(2); break;
+      case 3: GSPLAT_FWD_ROWS_P(3); break;
+      default: GSPLAT_FWD_ROWS_P(4); break;
+    }
+#undef GSPLAT_FWD_ROWS_P
+#undef GSPLAT_FWD_ROWS
+    return check_launch("rasterize_to_pixels_3dgs_forward");
+  }
   switch (ch) {
     case 1: raster_fwd_kernel<1><<<grid, bs, sm, s>>>(a, render_colors, render_alphas, last_ids); break;
     case 2: raster_fwd_kernel<2><<<grid, bs, sm, s>>>(a, render_colors, render_alphas, last_ids); break;
@@ -2053,13 +2395,10 @@ static int rasterize_bwd_impl(const float* means2d, const float* conics, const f
   const unsigned nb = static_cast<unsigned>(n_total);
   // one block per tile (block b: the tile of rank b in the heavy-first order)
   //
-  // Records in lanes wherever that kernel applies: whole 8x8 pixel blocks,
-  // staged colours, sums of signed gradients only, pixel centres exact in
-  // float under + 1 steps.
-  constexpr int kExactCentres = 1 << 22;
-  if (ch >= 1 && !v_means2d_abs && tile_size % 8 == 0 && image_width <= kExactCentres &&
-      image_height <= kExactCentres) {
-    const int bb = bwd_rows_batch(bs);
+  // Records in lanes wherever that kernel applies: staged colours, sums of
+  // signed gradients only
+  if (ch >= 1 && !v_means2d_abs && rows_kernels_apply(tile_size, image_width, image_height)) {
+    const int bb = bwd_rows_batch(bs, n_total);
     const size_t sm = bwd_rows_smem(ch, bs, bb);
 #define GSPLAT_BWD_ROWS(C)                                                                                     \
   raster_bwd_rows_kernel<C><<<nb, bs, sm, s>>>(a, bb, n_total, order, cost, render_alphas, last_ids,           \

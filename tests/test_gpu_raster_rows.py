@@ -1,10 +1,11 @@
-"""The rasterize backward with records in lanes (tile sides that are multiples
-of 8, one to four channels, no absolute gradients) against the oracle, where
-its groups of 16 records, its batches of 256 entries and its record classes
-meet: list lengths around 16 and 256, every tile side it takes, opacities over
-the 0.99 cap, ill-conditioned conics, opacities over 1 and non-finite records.
+"""The rasterizer kernels with records in lanes (tile sides 8, 16 and 24, one to
+four channels, no absolute gradients) against the oracle, where their groups of
+16 records, their batches of 128 and 256 entries, their record classes and the
+forward's pixel blocks meet: list lengths around 16, 128 and 256, every tile
+side, opacities over the 0.99 cap, ill-conditioned conics, opacities over 1,
+non-finite records, and grids on both sides of the forward's block sizes.
 
-Tolerance: the gradients' usual bar, 1e-3 of each element or of 1% of the
+Tolerance: images 1e-4 and exact last contributors as elsewhere; the gradients' usual bar, 1e-3 of each element or of 1% of the
 tensor's largest (both sides round every pixel's terms in float32; the sums
 run in another order).
 """
@@ -12,7 +13,7 @@ import numpy as np
 import pytest
 
 from _helpers import assert_close_rel, dev, gsplat, host
-from test_gpu_raster import GRAD_RTOL, _oracle_fwd, _raster_inputs, make_scene
+from test_gpu_raster import GRAD_RTOL, IMG_ATOL, _oracle_fwd, _raster_inputs, make_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +23,10 @@ def _check(oracle, s, W, H, ts, rng, finite=True):
     got = g.rasterize_to_pixels_3dgs_forward(_raster_inputs(s), W, H, ts)
     exp = _oracle_fwd(oracle, s, W, H, ts)
     np.testing.assert_array_equal(host(got["last_ids"]), exp["last_ids"])
+    for k in ("render_colors", "render_alphas"):
+        a, e = host(got[k]), exp[k]
+        np.testing.assert_array_equal(np.isfinite(a), np.isfinite(e), err_msg=k)
+        np.testing.assert_allclose(a[np.isfinite(e)], e[np.isfinite(e)], rtol=0, atol=IMG_ATOL, err_msg=k)
     v_rc = rng.normal(size=exp["render_colors"].shape).astype(np.float32)
     v_ra = rng.normal(size=exp["render_alphas"].shape).astype(np.float32)
     bwd = g.rasterize_to_pixels_3dgs_backward(
@@ -38,7 +43,7 @@ def _check(oracle, s, W, H, ts, rng, finite=True):
         assert_close_rel(a, e, GRAD_RTOL, k)
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 255, 256, 257, 529])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 127, 129, 255, 256, 257, 529])
 def test_list_lengths(oracle, n):
     """One tile whose list holds about n faint records (every group and batch remainder)."""
     rng = np.random.default_rng(n)
@@ -80,3 +85,28 @@ def test_ill_conditioned_and_non_finite_records(oracle):
     s["colors"].reshape(-1, 3)[250, 1] = np.inf
     s["colors"].reshape(-1, 3)[300, 2] = np.nan
     _check(oracle, s, W, H, 16, rng, finite=False)
+
+
+def test_forward_block_sizes_agree(oracle):
+    """The same image rendered as one of 1, 30 and 80 copies (12, 360 and 960
+    tiles: 4x4, 8x4 and 8x8 pixel blocks per wave) comes out bit for bit."""
+    import torch
+
+    rng = np.random.default_rng(3)
+    W, H, ts, n = 60, 47, 16, 800
+    s = make_scene(oracle, rng, 1, n, W, H, ts, 3, opac=(0.05, 0.999), scale=(1.0, 6.0))
+    _check(oracle, s, W, H, ts, rng)
+    g = gsplat()
+    one = _raster_inputs(s)
+    ref = g.rasterize_to_pixels_3dgs_forward(one, W, H, ts)
+    m = one["flatten_ids"].numel()
+    for copies in (30, 80):
+        many = {k: v.repeat(copies, *([1] * (v.dim() - 1))) for k, v in one.items() if k != "flatten_ids"}
+        step = torch.arange(copies, device="cuda", dtype=torch.int32)
+        many["tile_offsets"] = many["tile_offsets"] + (step * m)[:, None, None]
+        many["flatten_ids"] = (one["flatten_ids"][None] + (step * n)[:, None]).reshape(-1).contiguous()
+        got = g.rasterize_to_pixels_3dgs_forward(many, W, H, ts)
+        for k in ("render_colors", "render_alphas"):
+            assert torch.equal(got[k], ref[k].expand_as(got[k])), (copies, k)
+        want = torch.where(ref["render_alphas"][..., 0] > 0, ref["last_ids"] + (step * m)[:, None, None], 0)
+        assert torch.equal(got["last_ids"], want.to(got["last_ids"].dtype)), copies
