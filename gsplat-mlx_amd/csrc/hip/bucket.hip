@@ -24,12 +24,14 @@
 //     tile's base plus an LDS counter; the block's entries are dealt evenly
 //     over its threads (a Gaussian may cover thousands of tiles; ellipse
 //     lists: the entries of the round's tile rows);
-//  5. tile sort (one block per tile): the tile's pairs are sorted in LDS by a
-//     stable LSD radix sort on the depth bits, 8 bits a pass (passes whose
-//     digit is the same for the whole tile are skipped); a tile holding two
-//     equal depths is sorted again on (depth bits, flatten id), the id bytes
-//     as the low digits, so the order is the reference's whatever order the
-//     scatter left; the block writes the 64-bit ids and the flatten ids.
+//  5. tile sort (one block per tile): the tile's pairs are sorted in LDS by
+//     (depth bits, flatten id), so the order is the reference's whatever order
+//     the scatter left: one distribution over the range of the depth bits and
+//     a count within each bin. A tile whose depths crowd a bin takes a stable
+//     LSD radix sort on the depth bits instead, 8 bits a pass (passes whose
+//     digit is the same for the whole tile are skipped), sorted again on the
+//     id bytes and the depth bits where depths are equal. The block writes the
+//     64-bit ids and the flatten ids.
 //     Short lists are sorted by one launch over every list, each longer
 //     class by a launch of a larger instantiation; lists longer than the
 //     LDS holds (kBucketMaxList) are split by their most significant varying
@@ -107,9 +109,8 @@ __device__ __forceinline__ Segment segment_of(const BucketDims& d, int64_t lb) {
 // classes 0-2 (up to kSortCap[1..3]: <512, 8>, <512, 16>, <1024, 16>), each
 // sorted by its own launch, and class 3 (longer than LDS holds) by the split
 // sort below. At multiview_3m (lists of up to ~10,000) the tile sort takes
-// 2.25 ms this way against 2.78 ms with every list in the instantiation the
-// longest list needs; <512, 5> for the short lists and <1024, 8> for class 2
-// measured slower.
+// 1.39 ms this way; <1024, 8> for class 2 measured slower (1.57 ms), as does
+// every list in the instantiation the longest one needs.
 constexpr int kSortCap[4] = {256 * 10, 512 * 8, 512 * 16, 1024 * 16};
 constexpr int kSortClasses = 4;
 
@@ -727,7 +728,7 @@ __global__ void __launch_bounds__(kBucketBlock) bucket_scatter_kernel(const floa
   }
 }
 
-// 5. Tile sort. Elements live in LDS in list order; wave w holds the
+// 5. Tile sort, radix passes. Elements live in LDS in list order; wave w holds the
 // contiguous chunk [w R 64, (w + 1) R 64) in registers, R = ceil(n / (W 64))
 // rounds of 64, so every wave holds part of even a short list. One stable
 // pass on an 8-bit digit: wave-private running digit counts rank each wave's
@@ -833,6 +834,118 @@ struct TileSorter {
   }
 };
 
+// One-distribution sort of the n pairs at src (n <= B * ITEMS), written as
+// sort_range below; false, with nothing written, when a bin is crowded.
+//
+// The bins divide the keys' range evenly (8 per thread, two 16-bit counts a
+// word): they are counted by LDS atomics, their exclusive scan gives the bins'
+// first positions, and the elements go to LDS in bin order, any order within a
+// bin. An element's place is then its bin's first position plus the bin's
+// smaller (depth bits, flatten id) pairs, which it counts, so equal depths need
+// no pass of their own. Bins hold one to a few elements, and the whole costs
+// less than one of the radix sort's up to four passes, which were bound by the
+// ballots that rank equal digits: 72 -> 40 us at 5.4M entries in 4346 lists,
+// 38 -> 20 us at 1.06M in 5292, 2.03 -> 1.39 ms at 172M in 65280.
+//
+// Threads past the list count in words of their own, without a branch, so that
+// the atomics of a thread's elements overlap.
+constexpr int kBinCrowd = 48;
+
+template <int B, int ITEMS>
+__device__ __forceinline__ bool distribute(const uint2* src, int n, uint64_t hi, int64_t* out_ids, int32_t* out_flat,
+                                           uint2* s_kv, uint32_t* s_bins, uint32_t* s_dstart, uint32_t* s_bits) {
+  constexpr int W = B / kWave;
+  constexpr int kBins = W * 512, kBinWords = kBins / 2 / B;
+  static_assert(kBins == B * 8 && B * ITEMS < 65536, "bins per thread, 16-bit counts");
+  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+  // all loads in flight at once
+  uint2 e[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = r * B + t;
+    e[r] = j < n ? src[j] : make_uint2(0u, 0u);
+  }
+  if (t < 2) s_bits[t] = t ? ~0u : 0u;
+#pragma unroll
+  for (int q = 0; q < kBinWords; ++q) s_bins[q * B + t] = 0u;
+  __syncthreads();
+  uint32_t khi = 0u, klo = ~0u;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const bool in = r * B + t < n;
+    khi = max(khi, in ? e[r].x : 0u);
+    klo = min(klo, in ? e[r].x : ~0u);
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    khi = max(khi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(khi), off, kWave)));
+    klo = min(klo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(klo), off, kWave)));
+  }
+  if (lane == 0) {
+    atomicMax(&s_bits[0], khi);
+    atomicMin(&s_bits[1], klo);
+  }
+  __syncthreads();
+  uint32_t lowest = s_bits[1];
+  const uint32_t span = s_bits[0] - lowest;
+  if (span == 0 && n > kBinCrowd) return false;  // one depth: the radix sort on the ids
+  const int shift = max(0, (32 - __builtin_clz(span | 1u)) - (31 - __builtin_clz(static_cast<unsigned>(kBins))));
+  auto bin_of = [&](uint32_t key) { return (key - lowest) >> shift; };
+  auto bin_word = [&](int r, uint32_t b) { return r * B + t < n ? s_bins + (b >> 1) : s_dstart + 64 + lane; };
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t b = bin_of(e[r].x);
+    atomicAdd(bin_word(r, b), 1u << ((b & 1u) * 16u));
+  }
+  __syncthreads();
+  bool crowded = false;
+  uint32_t c[kBinWords], sum = 0;
+#pragma unroll
+  for (int q = 0; q < kBinWords; ++q) {
+    c[q] = s_bins[t * kBinWords + q];
+    const uint32_t a = c[q] & 0xffffu, b = c[q] >> 16;
+    crowded = crowded || max(a, b) > static_cast<uint32_t>(kBinCrowd);
+    sum += a + b;
+  }
+  const uint32_t inc = static_cast<uint32_t>(wave_inclusive_scan(static_cast<int>(sum)));
+  if (lane == kWave - 1) s_dstart[wave] = inc;
+  if (__syncthreads_or(crowded)) return false;
+  uint32_t run = inc - sum;
+#pragma unroll
+  for (int w = 0; w < W; ++w) run += w < wave ? s_dstart[w] : 0u;
+#pragma unroll
+  for (int q = 0; q < kBinWords; ++q) {
+    const uint32_t a = c[q] & 0xffffu;
+    s_bins[t * kBinWords + q] = run | ((run + a) << 16);
+    run += a + (c[q] >> 16);
+  }
+  __syncthreads();
+  asm volatile("" : "+v"(lowest));  // the bins are formed again, not kept in registers
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t b = bin_of(e[r].x), half = (b & 1u) * 16u;
+    const uint32_t pos = (atomicAdd(bin_word(r, b), 1u << half) >> half) & 0xffffu;
+    if (r * B + t < n) s_kv[pos] = e[r];
+  }
+  __syncthreads();
+  const uint16_t* last = reinterpret_cast<const uint16_t*>(s_bins);  // one past each bin, once placed
+  for (int j = t; j < n; j += B) {
+    const uint2 v = s_kv[j];
+    const uint32_t b = bin_of(v.x);
+    const int b0 = b > 0 ? last[b - 1] : 0, b1 = last[b];
+    int pos = b0;
+    if (b1 - b0 > 1) {
+      for (int i = b0; i < b1; ++i) {
+        const uint2 o = s_kv[i];
+        pos += (o.x < v.x || (o.x == v.x && o.y < v.y)) ? 1 : 0;
+      }
+    }
+    out_ids[pos] = static_cast<int64_t>(hi | v.x);
+    out_flat[pos] = static_cast<int32_t>(v.y);
+  }
+  return true;
+}
+
 // The n (depth bits, flatten id) pairs at src sorted in LDS (the shared
 // arrays of the calling kernel) and written as ids hi | depth bits and
 // flatten ids at out_ids / out_flat. Every input is read before any output
@@ -845,6 +958,14 @@ __device__ __forceinline__ void sort_range(const uint2* src, int64_t len, uint64
   if (len <= 0 || len > S::CAP) return;  // block-uniform
   const int n = static_cast<int>(len);
   const int t = threadIdx.x;
+  // half the items where the list fits: no element slots without an element
+  constexpr int kHalf = ITEMS / 2;
+  if (n <= B * kHalf) {
+    if (distribute<B, kHalf>(src, n, hi, out_ids, out_flat, s_kv, s_wcnt, s_dstart, s_bits)) return;
+  } else {
+    if (distribute<B, ITEMS>(src, n, hi, out_ids, out_flat, s_kv, s_wcnt, s_dstart, s_bits)) return;
+  }
+  // Depths of very uneven spread or many equal ones: radix passes.
   if (t < 4) s_bits[t] = (t & 1) ? ~0u : 0u;
   __syncthreads();
   // the bits that vary over the list: passes on digits every element shares
@@ -977,10 +1098,18 @@ struct TileSortLds {
   uint32_t bits[4];  // OR and AND of the keys, OR and AND of the ids
 };
 
+// Waves per SIMD that the LDS admits: the register budget of the sorts. What
+// that budget spills is the radix passes' arrays, off the usual path (4346
+// lists of 1241 entries on average: 50 us at four waves per SIMD, 44 at five,
+// 40 at six).
+constexpr int tile_sort_waves(int b, int items) {
+  return static_cast<int>(kLdsBytes / (b * items * 8 + b / kWave * 1024 + 1040)) * b / kWave / 4;
+}
+
 // Block b sorts list b and writes its tile offset (every list; lists longer
 // than this instantiation holds are left to the class kernels).
 template <int B, int ITEMS>
-__global__ void __launch_bounds__(B) bucket_tile_sort_kernel(const uint2* __restrict__ pairs,
+__global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(tile_sort_waves(B, ITEMS)))) bucket_tile_sort_kernel(const uint2* __restrict__ pairs,
                                                              const int32_t* __restrict__ tile_start, int64_t n_lists,
                                                              int64_t n_isects, const int64_t* __restrict__ m_dev,
                                                              int64_t n_tiles, int tile_bits,
@@ -998,7 +1127,7 @@ __global__ void __launch_bounds__(B) bucket_tile_sort_kernel(const uint2* __rest
 // Block b sorts list b of one long class (the tile pass's binning); blocks
 // past the class's size exit at once.
 template <int B, int ITEMS>
-__global__ void __launch_bounds__(B) bucket_tile_sort_class_kernel(const uint2* __restrict__ pairs,
+__global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(tile_sort_waves(B, ITEMS)))) bucket_tile_sort_class_kernel(const uint2* __restrict__ pairs,
                                                                    const int32_t* __restrict__ tile_start,
                                                                    int64_t n_lists, int64_t n_isects,
                                                                    const int64_t* __restrict__ m_dev, int64_t n_tiles,
