@@ -44,3 +44,31 @@ def test_one_tile(n, kind):
     ids = host(out["isect_ids"]).astype(np.uint64)
     np.testing.assert_array_equal((ids & 0xFFFFFFFF).astype(np.uint32), bits[order])
     assert host(out["tile_offsets"]).ravel().tolist() == [0]
+
+
+@pytest.mark.parametrize("images", [1, 2, 7, 32, 33])
+def test_images_start_after_the_earlier_ones(images):
+    """Offsets and lists over several images (a tile pass block per image up to
+    32 of them, one block for all beyond), one image empty, against a numpy
+    enumeration."""
+    rng = np.random.default_rng(images)
+    n, tw, th = 300, 5, 3
+    m = rng.uniform(-10, 90, (images, n, 2)).astype(np.float32)
+    r = rng.integers(0, 30, (images, n, 2)).astype(np.int32)
+    if images > 1:
+        r[images // 2] = 0
+    d = rng.uniform(0.2, 9.0, (images, n)).astype(np.float32)
+    g = gsplat()
+    out = g.intersect_tile_offsets_forward({"means2d": dev(m), "radii": dev(r), "depths": dev(d)}, images, 16, tw, th)
+    lo = np.clip(np.floor((m - r) / 16), 0, [tw, th]).astype(int)
+    hi = np.clip(np.ceil((m + r) / 16), 0, [tw, th]).astype(int)
+    rows = []
+    for i in range(images):
+        for k in range(n):
+            if (r[i, k] > 0).all():
+                rows += [(i * tw * th + y * tw + x, d[i, k].view(np.uint32), i * n + k)
+                         for y in range(lo[i, k, 1], hi[i, k, 1]) for x in range(lo[i, k, 0], hi[i, k, 0])]
+    rows = np.array(sorted(rows), np.int64).reshape(-1, 3)
+    np.testing.assert_array_equal(host(out["flatten_ids"]), rows[:, 2])
+    np.testing.assert_array_equal(host(out["tile_offsets"]).ravel(), np.searchsorted(rows[:, 0], np.arange(images * tw * th)))
+    assert out["isect_ids"].numel() == len(rows)
