@@ -872,7 +872,9 @@ struct TileSorter {
 };
 
 // One-distribution sort of the n pairs at src (n <= B * ITEMS), written as
-// sort_range below; false, with nothing written, when a bin is crowded.
+// sort_range below; false, with nothing written, when a bin is crowded. False
+// comes behind a barrier after every read of the shared arrays, so the caller
+// may write them at once.
 //
 // The bins divide the keys' range evenly (8 per thread, two 16-bit counts a
 // word): they are counted by LDS atomics, their exclusive scan gives the bins'
@@ -925,7 +927,10 @@ __device__ __forceinline__ bool distribute(const uint2* src, int n, uint64_t hi,
   __syncthreads();
   uint32_t lowest = s_bits[1];
   const uint32_t span = s_bits[0] - lowest;
-  if (span == 0 && n > kBinCrowd) return false;  // one depth: the radix sort on the ids
+  if (span == 0 && n > kBinCrowd) {  // one depth: the radix sort on the ids
+    __syncthreads();                 // every wave has read s_bits
+    return false;
+  }
   const int shift = max(0, (32 - __builtin_clz(span | 1u)) - (31 - __builtin_clz(static_cast<unsigned>(kBins))));
   auto bin_of = [&](uint32_t key) { return (key - lowest) >> shift; };
   auto bin_word = [&](int r, uint32_t b) { return r * B + t < n ? s_bins + (b >> 1) : s_dstart + 64 + lane; };

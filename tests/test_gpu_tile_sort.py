@@ -46,6 +46,29 @@ def test_one_tile(n, kind):
     assert host(out["tile_offsets"]).ravel().tolist() == [0]
 
 
+@pytest.mark.parametrize("per_tile,side,planes", [
+    ([0, 1, 48, 49, 64, 300, 1280, 1281, 2560], 40, 1), ([2561, 4096, 5000, 8192, 9000, 16384], 16, 1),
+    ([16385, 17000], 2, 1), ([20000, 24000], 4, 4)])
+def test_a_frame_of_one_depth(per_tile, side, planes):
+    """A plane facing the camera: the entries of every tile have the same depth
+    bits, at the lengths of every instantiation and in many tiles, so that
+    blocks share CUs; and lists past 16384 entries of four such planes, each
+    plane a run of its own. The order is (depth, flatten id)."""
+    lengths = np.resize(np.array(per_tile), side * side)
+    rng = np.random.default_rng(lengths.size)
+    tile = rng.permutation(np.repeat(np.arange(side * side), lengths))
+    n = tile.size
+    m = (np.stack([tile % side, tile // side], -1) * 16 + 8).astype(np.float32)[None]
+    d = (2.0 ** rng.integers(0, planes, n)).astype(np.float32)
+    out = gsplat().intersect_tile_offsets_forward(
+        {"means2d": dev(m), "radii": dev(np.full((1, n, 2), 3, np.int32)), "depths": dev(d[None])}, 1, 16, side, side)
+    order = np.lexsort((np.arange(n), d, tile))
+    np.testing.assert_array_equal(host(out["flatten_ids"]), order.astype(np.int32))
+    ids = (tile[order].astype(np.int64) << 32) | d[order].view(np.uint32)
+    np.testing.assert_array_equal(host(out["isect_ids"]), ids)
+    np.testing.assert_array_equal(host(out["tile_offsets"]).ravel(), np.cumsum(lengths) - lengths)
+
+
 @pytest.mark.parametrize("images", [1, 2, 7, 32, 33])
 def test_images_start_after_the_earlier_ones(images):
     """Offsets and lists over several images (a tile pass block per image up to
