@@ -1438,7 +1438,9 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
       for (int c = 0; c < CH; ++c) bg_dot += bg[c] * v_rc[c];
     }
     const float coef = T_final * v_ra + -T_final * bg_dot;
-    bool rc_finite = fabsf(T_final) <= 3.402823466e38f;
+    // all of the wave's pixel values finite: then a record that a pixel does
+    // not take adds -0 v_alpha = 0 without a select (levels 0 and 1 below)
+    bool rc_finite = fabsf(T_final) <= 3.402823466e38f && fabsf(coef) <= 3.402823466e38f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) rc_finite = rc_finite && fabsf(v_rc[c]) <= 3.402823466e38f;
     wave_rc_finite = __ballot(!rc_finite) == 0;

@@ -110,3 +110,38 @@ def test_forward_block_sizes_agree(oracle):
             assert torch.equal(got[k], ref[k].expand_as(got[k])), (copies, k)
         want = torch.where(ref["render_alphas"][..., 0] > 0, ref["last_ids"] + (step * m)[:, None, None], 0)
         assert torch.equal(got["last_ids"], want.to(got["last_ids"].dtype)), copies
+
+
+def _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra):
+    """The backward's non-finite gradients are the oracle's: a pixel's values
+    reach only the Gaussians that it takes."""
+    exp = _oracle_fwd(oracle, s, W, H, 16)
+    bwd = gsplat().rasterize_to_pixels_3dgs_backward(
+        _raster_inputs(s), {"render_alphas": dev(exp["render_alphas"]), "last_ids": dev(exp["last_ids"])},
+        {"v_render_colors": dev(v_rc), "v_render_alphas": dev(v_ra)}, W, H, 16)
+    want = oracle.raster_backward(s["means2d"], s["conics"], s["colors"], s["opacities"], s["tile_offsets"],
+                                  s["flatten_ids"], W, H, 16, exp["render_alphas"], exp["last_ids"], v_rc, v_ra,
+                                  backgrounds=s["backgrounds"])
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        a, e = host(bwd[k]), want[k]
+        np.testing.assert_array_equal(np.isfinite(a), np.isfinite(e), err_msg=k)
+        fin = np.isfinite(e)
+        assert fin.mean() > 0.8, k
+        assert_close_rel(np.where(fin, a, 0), np.where(fin, e, 0), GRAD_RTOL, k)
+    return want
+
+
+@pytest.mark.parametrize("opac", [(0.05, 0.9), (0.5, 1.0)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_non_finite_alpha_cotangents_stay_local(oracle, value, opac):
+    """NaN and inf in the alpha cotangents of single pixels whose colour
+    cotangents are finite, in groups without and with records over the cap."""
+    rng = np.random.default_rng(29)
+    W = H = 96
+    s = make_scene(oracle, rng, 1, 1200, W, H, 16, 3, opac=opac)
+    v_rc = rng.normal(size=(1, H, W, 3)).astype(np.float32)
+    v_ra = rng.normal(size=(1, H, W, 1)).astype(np.float32)
+    v_ra[0, 40, 41] = value
+    v_ra[0, 70, 12] = -value
+    want = _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
+    assert not np.isfinite(want["v_opacities"]).all()
