@@ -1637,7 +1637,11 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
               S[h] += vs[h];
               Hx[h] = __builtin_fmaf(vs[h], dx[p], Hx[h]);
             }
-            Hxx = __builtin_fmaf(vs[0] + vs[1], dx[p] * dx[p], Hxx);
+            if constexpr (kCareful) {  // the means may lie so far that dx dx overflows, with vs 0
+              Hxx = __builtin_fmaf((vs[0] + vs[1]) * dx[p], dx[p], Hxx);
+            } else {
+              Hxx = __builtin_fmaf(vs[0] + vs[1], dx[p] * dx[p], Hxx);
+            }
           }
         }
       };

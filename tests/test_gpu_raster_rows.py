@@ -145,3 +145,21 @@ def test_non_finite_alpha_cotangents_stay_local(oracle, value, opac):
     v_ra[0, 70, 12] = -value
     want = _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
     assert not np.isfinite(want["v_opacities"]).all()
+
+
+def test_far_finite_means_give_no_gradient(oracle):
+    """Finite means so far away that the square of their distance overflows:
+    never culled, taken by no pixel, and without a gradient."""
+    rng = np.random.default_rng(31)
+    W = H = 48
+    s = make_scene(oracle, rng, 1, 500, W, H, 16, 3, opac=(0.05, 0.6), scale=(1.0, 4.0))
+    mean = s["means2d"].reshape(-1, 2)
+    mean[100] = [1.0e31, 20.0]
+    mean[222] = [20.0, -3.0e37]
+    mean[333] = [-2.0e20, 5.0e19]
+    s["conics"].reshape(-1, 3)[333] = [0.2, 0.199999, 0.2]
+    v_rc = rng.normal(size=(1, H, W, 3)).astype(np.float32)
+    v_ra = rng.normal(size=(1, H, W, 1)).astype(np.float32)
+    want = _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
+    assert all(np.isfinite(want[k]).all() for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"))
+    assert (want["v_conics"].reshape(-1, 3)[[100, 222, 333]] == 0).all()
