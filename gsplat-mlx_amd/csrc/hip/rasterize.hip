@@ -149,7 +149,9 @@ __device__ __forceinline__ float exp_alpha_bounded(float y) {
 //   then keeps sigma below 2e9, so the exponential needs no clamp.
 // - kCappedRecord clear: also an opacity up to 0.99, so alpha = o exp(-sigma)
 //   never meets the cap.
-constexpr uint32_t kNonFiniteRecord = 1u << 31;  // a non-finite mean or staged colour (backward)
+// - kNonFiniteRecord: a non-finite staged colour, in the backward also a
+//   non-finite mean (records in lanes: a colour beyond kTameColor).
+constexpr uint32_t kNonFiniteRecord = 1u << 31;
 constexpr uint32_t kGeneralRecord = 1u << 30;
 constexpr uint32_t kCappedRecord = 1u << 29;
 
@@ -1322,6 +1324,13 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 // 114 -> 81 us at 512x512. About 120 VGPRs hold four evaluations in flight
 // (their scans interleave without wait states); at five waves per SIMD (96
 // VGPRs) the loop spills, 293 us, and unrolled further it does at four.
+//
+// kTameColor, kTameBuffer: bounds of the colours (and their cotangents) and of
+// the entering buffer for which levels 0 and 1 run. Up to four products of a
+// colour and a cotangent, their sums weighted by at most 1 in all, the entering
+// buffer and its 1 / (1 - alpha) <= 100 fold then stay below 1e33, so v_alpha is
+// finite at every pixel.
+constexpr float kTameColor = 1.0e15f, kTameBuffer = 1.0e30f;
 constexpr int kNeutral = 40;  // entries of the neutral state: columns 0-7 of two rows 32 apart
 
 template <int CH>
@@ -1413,7 +1422,7 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
 
   store_wave_rects(s_rect, n_waves, a.ts, tx, ty);
   int wave_last;
-  bool wave_rc_finite;
+  bool wave_tame;
   {
     int qx, qy;
     lane_pixel(t, a.ts, &qx, &qy);
@@ -1438,12 +1447,12 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
       for (int c = 0; c < CH; ++c) bg_dot += bg[c] * v_rc[c];
     }
     const float coef = T_final * v_ra + -T_final * bg_dot;
-    // all of the wave's pixel values finite: then a record that a pixel does
-    // not take adds -0 v_alpha = 0 without a select (levels 0 and 1 below)
-    bool rc_finite = fabsf(T_final) <= 3.402823466e38f && fabsf(coef) <= 3.402823466e38f;
+    // all of the wave's pixel values tame: then a record that a pixel does not
+    // take adds -0 v_alpha = 0 without a select (levels 0 and 1 below)
+    bool rc_tame = fabsf(T_final) <= 3.402823466e38f && fabsf(coef) <= kTameBuffer;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) rc_finite = rc_finite && fabsf(v_rc[c]) <= 3.402823466e38f;
-    wave_rc_finite = __ballot(!rc_finite) == 0;
+    for (int c = 0; c < CH; ++c) rc_tame = rc_tame && fabsf(v_rc[c]) <= kTameColor;
+    wave_tame = __ballot(!rc_tame) == 0;
     wave_last = last_rel;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) wave_last = max(wave_last, __shfl_xor(wave_last, off, kWave));
@@ -1483,7 +1492,7 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
       tail[GW - 4] = __int_as_float(r_g);
       bool rec_finite = fabsf(r_xy.x) <= 3.402823466e38f && fabsf(r_xy.y) <= 3.402823466e38f;
 #pragma unroll
-      for (int c = 0; c < CH; ++c) rec_finite = rec_finite && fabsf(r_col[c]) <= 3.402823466e38f;
+      for (int c = 0; c < CH; ++c) rec_finite = rec_finite && fabsf(r_col[c]) <= kTameColor;
       tail[GW - 3] = __uint_as_float(r_mask | (rec_finite ? 0u : kNonFiniteRecord));
 #pragma unroll
       for (int i = 0; i < RW - 4; i += 4)
@@ -1647,7 +1656,7 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
       };
       int level = 0;
       if (__ballot(live && (bits & kCappedRecord)) != 0) level = 1;
-      if (!wave_rc_finite || __ballot(live && (bits & (kGeneralRecord | kNonFiniteRecord))) != 0) level = 2;
+      if (!wave_tame || __ballot(live && (bits & (kGeneralRecord | kNonFiniteRecord))) != 0) level = 2;
       if (level == 0) {
         walk(std::integral_constant<int, 0>{});
       } else if (level == 1) {

@@ -163,3 +163,20 @@ def test_far_finite_means_give_no_gradient(oracle):
     want = _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
     assert all(np.isfinite(want[k]).all() for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"))
     assert (want["v_conics"].reshape(-1, 3)[[100, 222, 333]] == 0).all()
+
+
+@pytest.mark.parametrize("color,cotangent,background", [(1.0e30, 1.0e20, 0.1), (0.5, 1.0e20, 1.0e30), (1.0e34, 1.0e12, 0.1)])
+def test_overflowing_products_stay_local(oracle, color, cotangent, background):
+    """Finite colours, backgrounds and cotangents whose products overflow at two
+    pixels, there beyond 1e43, so that every order of the products with T > 1e-4
+    overflows, and stay below 1e36 at the others."""
+    rng = np.random.default_rng(37)
+    W = H = 96
+    s = make_scene(oracle, rng, 1, 1200, W, H, 16, 3)
+    s["colors"][0, [5, 700]] = color
+    s["backgrounds"][:] = background
+    v_rc = rng.normal(size=(1, H, W, 3)).astype(np.float32)
+    v_rc[0, 40, 41] = cotangent
+    v_rc[0, 70, 12] = -cotangent
+    v_ra = rng.normal(size=(1, H, W, 1)).astype(np.float32)
+    _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
