@@ -493,7 +493,6 @@ struct RowBlock {
   static constexpr int HS = P == 64 ? 4 : 1;          // rows between a lane's two
   static __device__ __forceinline__ int x0(int g) { return P == 64 ? 0 : (g & 1) * NX; }
   static __device__ __forceinline__ int y0(int g) { return P == 64 ? g : (g >> 1) * 2; }
-  static __host__ __device__ constexpr int waves(int ts) { return ts * ts / P; }
   static __device__ __forceinline__ PixRect rect(int w, int ts, int tx, int ty) {
     const int bpr = ts / BX;
     PixRect r;
@@ -505,7 +504,8 @@ struct RowBlock {
   }
 };
 
-// Forward with records in lanes: tile sides 8, 16 and 24, one to four channels.
+// Forward with records in lanes: tile sides 8 and 16, one to four channels
+// (fwd_rows_faster says where).
 // Staging and culling are raster_fwd_kernel's, and so are every alpha,
 // transmittance and sum, bit for bit. A wave takes the records that may touch
 // its pixels in groups of 16, in two steps:
@@ -536,7 +536,7 @@ constexpr int kRowsBatch = 256;
 constexpr int kRowsSmallBatch = 128;
 
 template <int CH, int P>
-__global__ void __launch_bounds__(576) raster_fwd_rows_kernel(RasterArgs a, int BB, int split,
+__global__ void __launch_bounds__(256) raster_fwd_rows_kernel(RasterArgs a, int BB, int split,
                                                                float* __restrict__ render_colors,
                                                                float* __restrict__ render_alphas,
                                                                int32_t* __restrict__ last_ids) {
@@ -1290,9 +1290,10 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 }
 #undef GSPLAT_ROW_STEP
 
-// Backward with records in lanes: tile sides 8, 16 and 24, one to four channels, no absolute gradients (the training path). Block, schedule,
-// staging and flush are raster_bwd_kernel's; a wave still owns an 8x8 block of
-// pixels, but evaluates 16 records at a time: lane l holds record l % 16 of
+// Backward with records in lanes: tile sides 8, 16 and 24, one to four channels,
+// no absolute gradients (the training path). Block, schedule, staging and flush
+// are raster_bwd_kernel's; a wave still owns an 8x8 block of pixels, but
+// evaluates 16 records at a time: lane l holds record l % 16 of
 // the group (in list order, back to front) and the pixel rows l / 16 and
 // l / 16 + 4, and steps over the 8 columns.
 // - A record's gradient sums stay in its lane's registers over all the wave's
@@ -2058,6 +2059,31 @@ bool rows_kernels_apply(int ts, int width, int height) {
   return (ts == 8 || ts == 16 || ts == 24) && width <= (1 << 22) && height <= (1 << 22);
 }
 
+// Where the forward with records in lanes is the faster one (the results are
+// the same bits). A group costs the same for one record as for 16, so short
+// lists are better off in the kernel with pixels in lanes, whose smaller LDS also
+// keeps more blocks resident: the lines lie higher once the tiles come in more
+// than one round of resident blocks. Times of the kernel with pixels in lanes over
+// this one's, three channels, scenes of 1000 to 1,000,000 Gaussians:
+// - side 16, 475 tiles: 0.95 at 4 entries per tile, 1.00-1.01 at 8 to 14, 1.2
+//   at 20 to 40. 784 tiles (two blocks each, more than are resident): 0.85 at
+//   19, 0.94-0.97 at 30 to 38, 1.13 at 62.
+// - 960 to 1200 tiles: 0.96-1.00 at 16 to 18, 1.0-1.06 at 22 to 30. 1900 to 18,900
+//   tiles: 0.8-0.9 up to 35, 0.91-1.09 at 40 to 55, 0.97-1.07 at 65 to 95, 1.0-1.2
+//   beyond (evenly spread lists of about 145 entries, a batch and a bit: 0.93-0.97).
+// - four channels (colours and entries in separate words): 0.97-1.06 at 1024
+//   tiles and 17 to 169 entries, 1.10-1.14 beyond; 0.95-1.05 on larger grids.
+// - side 8 (a wave per block): 1.04-1.4 up to 1900 tiles, 1.1-1.25 at 4096 from
+//   34 on (0.94 at 4), 0.64-1.0 on most larger grids (1.05-1.14 on two). Side 24
+//   (9 waves, 3 blocks per CU by LDS): 0.7-1.0 nearly everywhere.
+bool fwd_rows_faster(int ts, int ch, int64_t n_tiles, int64_t per_tile) {
+  if (ts == 24) return false;
+  if (ts == 8) return n_tiles <= 4096 && per_tile >= (n_tiles <= 2048 ? 8 : 32);
+  if (n_tiles <= 800) return per_tile >= (n_tiles <= 512 ? 12 : 48);
+  if (n_tiles <= 1536) return per_tile >= (ch < 4 ? 24 : 128);  // 6 blocks on each of 256 CUs
+  return ch < 4 && per_tile >= 64;
+}
+
 // raster_fwd_rows_kernel: records, alphas, colours, wave rectangles, entries and
 // record lists.
 size_t fwd_rows_smem(int ch, int n_waves, int pixels, int bb) {
@@ -2295,10 +2321,11 @@ static int rasterize_fwd_impl(const float* means2d, const float* conics, const f
   const int ch = channels <= 4 ? channels : 0;
   const size_t sm = fwd_smem(ch, bs);
   KernelTimer timer("raster_fwd", s);
-  // records in lanes wherever that kernel applies (pixel centres exact in
-  // float under + 1 steps), with smaller pixel blocks on small grids
+  // records in lanes where that kernel applies and is the faster one, with
+  // smaller pixel blocks on small grids
   const int64_t n_total = I * tile_width * static_cast<int64_t>(tile_height);
-  if (ch >= 1 && rows_kernels_apply(tile_size, image_width, image_height)) {
+  if (ch >= 1 && rows_kernels_apply(tile_size, image_width, image_height) &&
+      fwd_rows_faster(tile_size, ch, n_total, n_isects / n_total)) {
     const int pixels = tile_size != 16 || n_total > 800 ? 64 : (n_total > 320 ? 32 : 16);
     const int split = 64 / pixels;
     const int n_waves = tile_size * tile_size / 64;

@@ -180,3 +180,58 @@ def test_overflowing_products_stay_local(oracle, color, cotangent, background):
     v_rc[0, 70, 12] = -cotangent
     v_ra = rng.normal(size=(1, H, W, 1)).astype(np.float32)
     _check_backward_stays_local(oracle, s, W, H, v_rc, v_ra)
+
+
+def _pad_lists(s, pad):
+    """The scene with `pad` entries of an added Gaussian of opacity 0 at the end of
+    every tile's list: the same image and gradients, longer lists."""
+    n = s["opacities"].shape[1]
+    offs = s["tile_offsets"].reshape(-1).astype(np.int64)
+    ends = np.append(offs[1:], s["flatten_ids"].size)
+    at = np.repeat(ends, pad)
+    out = dict(s)
+    out["flatten_ids"] = np.insert(s["flatten_ids"], at, n).astype(np.int32)
+    out["tile_offsets"] = (offs + np.arange(offs.size) * pad).astype(np.int32).reshape(s["tile_offsets"].shape)
+    for k in ("means2d", "conics", "colors", "opacities"):
+        last = np.ones_like(s[k][:, :1]) * (0.0 if k == "opacities" else 1.0)
+        out[k] = np.concatenate([s[k], last.astype(np.float32)], 1)
+    return out
+
+
+@pytest.mark.parametrize("ts,C,W,H,pads", [
+    (16, 3, 64, 48, [40]), (16, 4, 256, 240, [40]), (16, 3, 448, 400, [60]), (16, 4, 512, 496, [140]),
+    (16, 1, 512, 496, [40]), (16, 3, 720, 560, [100, 300]), (16, 4, 720, 560, [100]), (8, 2, 200, 160, [40]),
+    (8, 3, 400, 400, [40]), (8, 3, 600, 520, [140]), (24, 3, 120, 96, [40]), (24, 4, 700, 720, [40]),
+    (24, 2, 700, 720, [300])])
+def test_kernels_for_short_and_long_lists_agree(oracle, ts, C, W, H, pads):
+    """Both sides of the lines by entries per tile, on grids of each of the rules'
+    sizes: short lists, and the same lists lengthened past the line by entries
+    that no pixel takes. The images are the same bits; the gradients differ by
+    the order of their sums."""
+    import torch
+
+    rng = np.random.default_rng(W + C)
+    tiles = -(-W // ts) * -(-H // ts)
+    n = max(tiles if ts == 8 else 2 * tiles, 60)
+    s = make_scene(oracle, rng, 1, n, W, H, ts, C, opac=(0.05, 0.999), scale=(0.5, 2.5))
+    v_rc = dev(rng.normal(size=(1, H, W, C)).astype(np.float32))
+    v_ra = dev(rng.normal(size=(1, H, W, 1)).astype(np.float32))
+    g = gsplat()
+    fwd, bwd = [], []
+    for x in [s] + [_pad_lists(s, pad) for pad in pads]:
+        inp = _raster_inputs(x)
+        f = g.rasterize_to_pixels_3dgs_forward(inp, W, H, ts)
+        bwd.append(g.rasterize_to_pixels_3dgs_backward(
+            inp, {"render_alphas": f["render_alphas"], "last_ids": f["last_ids"]},
+            {"v_render_colors": v_rc, "v_render_alphas": v_ra}, W, H, ts))
+        first = inp["tile_offsets"].repeat_interleave(ts, 1).repeat_interleave(ts, 2)[:, :H, :W]
+        f["last_ids"] = torch.where(f["last_ids"] > 0, f["last_ids"] - first, 0)
+        fwd.append(f)
+    for f, b in zip(fwd[1:], bwd[1:]):
+        for k in ("render_colors", "render_alphas"):
+            assert torch.equal(f[k], fwd[0][k]), k
+        taken = fwd[0]["render_alphas"][..., 0] > 0
+        assert torch.equal(f["last_ids"][taken], fwd[0]["last_ids"][taken])
+        for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+            assert (b[k][:, n] == 0).all(), k
+            assert_close_rel(host(b[k][:, :n]), host(bwd[0][k]), GRAD_RTOL, k)
