@@ -12,11 +12,12 @@
 // Backward: one block per tile, dispatched heaviest tile first, replays the
 // tile's list back-to-front from its largest last_id, rebuilding
 // transmittance per pixel, and each batch ends with one atomic per (record,
-// nonzero component). raster_bwd_rows_kernel (the training path) keeps 16
-// records in a wave's lanes and runs the pixel recurrences across them;
-// raster_bwd_kernel (other tile sides, more than four channels, absolute
-// gradients) keeps pixels in lanes and sums each record's partial gradients
-// over the wave by a transposed DPP/permlane reduction into per-wave LDS slots.
+// nonzero component). raster_bwd_rows_kernel keeps 16 records in a wave's lanes
+// and runs the pixel recurrences across them; raster_bwd_kernel (short lists,
+// other tile sides, more than four channels, absolute gradients) keeps pixels in
+// lanes and sums each record's partial gradients over the wave by a transposed
+// DPP/permlane reduction into per-wave LDS slots. The forward has the same two
+// forms: raster_fwd_rows_kernel and raster_fwd_kernel.
 //
 // Per-pixel math follows gsplat_core/gsplat_rasterize.cpp:291-368 (forward)
 // and :432-554 (backward) operation for operation; the Gaussian falloff and
@@ -1291,9 +1292,9 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 #undef GSPLAT_ROW_STEP
 
 // Backward with records in lanes: tile sides 8, 16 and 24, one to four channels,
-// no absolute gradients (the training path). Block, schedule, staging and flush
-// are raster_bwd_kernel's; a wave still owns an 8x8 block of pixels, but
-// evaluates 16 records at a time: lane l holds record l % 16 of
+// no absolute gradients, lists long enough (bwd_rows_faster). Block, schedule,
+// staging and flush are raster_bwd_kernel's; a wave still owns an 8x8 block of
+// pixels, but evaluates 16 records at a time: lane l holds record l % 16 of
 // the group (in list order, back to front) and the pixel rows l / 16 and
 // l / 16 + 4, and steps over the 8 columns.
 // - A record's gradient sums stay in its lane's registers over all the wave's
@@ -2084,6 +2085,28 @@ bool fwd_rows_faster(int ts, int ch, int64_t n_tiles, int64_t per_tile) {
   return ch < 4 && per_tile >= 64;
 }
 
+// The same for the backward (also by the block's registers: 4 blocks per CU of
+// side 16, one of side 24, against 6 and 2):
+// - side 16, 475 tiles: 0.87-0.95 at 4 to 8 entries per tile, 0.95-1.27 at 12 to
+//   21. 960 and 1024 tiles: 0.87-0.95 up to 18, 0.99-1.06 at 25, 1.06-1.08 at 35.
+//   1125 to 18,900 tiles: 0.55-0.9 up to 30, 0.92-1.2 at 55 to 70, 0.95-1.12 at 72
+//   to 82, 1.1-1.35 beyond.
+// - side 8: 1.0-1.25 up to 3072 tiles, 1.06-1.18 at 4096 from 34 on (0.85 at 4),
+//   on larger grids 0.9-1.0 up to 96 and 1.0-1.1 beyond; four channels, which
+//   spill, 0.7-1.06 from 4096 tiles on.
+// - side 24: 1.04-1.5 up to 663 tiles from 33 on (0.6-0.75 at 12 to 22); from 850
+//   tiles on 0.5-1.0 up to 180 and 1.0-1.3 beyond, with four channels 1.02-1.7
+//   from 40 on.
+bool bwd_rows_faster(int ts, int ch, int64_t n_tiles, int64_t per_tile) {
+  if (ts == 24) return per_tile >= (n_tiles <= 768 || ch == 4 ? 32 : 256);
+  if (ts == 8) {
+    if (n_tiles <= 2048) return per_tile >= (ch < 4 ? 8 : 32);
+    return ch < 4 && per_tile >= (n_tiles <= 4096 ? 32 : 128);
+  }
+  if (n_tiles <= 1024) return per_tile >= (n_tiles <= 512 ? 16 : 32);
+  return per_tile >= 80;
+}
+
 // raster_fwd_rows_kernel: records, alphas, colours, wave rectangles, entries and
 // record lists.
 size_t fwd_rows_smem(int ch, int n_waves, int pixels, int bb) {
@@ -2094,11 +2117,21 @@ size_t fwd_rows_smem(int ch, int n_waves, int pixels, int bb) {
 
 // raster_bwd_rows_kernel: accumulators, pixel cotangents and state, records, wave
 // rectangles and record lists, in the kernel's order.
-// Batches: 256 entries leave the fewest barriers and flushes (1M Gaussians,
-// 4346 tiles: 232 us against 242 at 128); where all tiles are resident at once
-// (4 blocks on each of 256 CUs), 128 shorten the heaviest tiles' start (100,000
-// Gaussians, 1024 tiles: 79.6 us against 82.2).
-int bwd_rows_batch(int bs, int64_t n_tiles) { return std::min(bs, n_tiles <= 1024 ? kRowsSmallBatch : kRowsBatch); }
+// Batches: 256 entries leave the fewest barriers and flushes (1M Gaussians, 4346
+// tiles of 1245 entries: 232 us against 242 at 128). Of side 16, 128 keep as many
+// blocks resident (by registers, 4 per CU) and suit shorter lists: 1.0 to 1.16
+// times the speed of 256 at 70 to 250 entries per tile, 0.86 to 1.0 from 270 on.
+// With four channels LDS admits 3 blocks of 256 entries or 4 of 128: 1.0 to 1.2
+// times the speed.
+// Up to 1024 tiles 128, though 256 are 1.0 to 1.3 times as fast there (side 24
+// up to 1.4): tiles add to a Gaussian by float atomics, in no fixed order, and
+// with 256 entries this showed more. 10,000 Gaussians at 256x256: three quaternion
+// gradients of one Gaussian, all cancellation, differed by 3e-4 between a third
+// of 120 runs; with 128 none by 1e-4.
+int bwd_rows_batch(int ts, int bs, int ch, int64_t n_tiles, int64_t per_tile) {
+  const bool small = n_tiles <= 1024 || (ts == 16 && (ch == 4 || per_tile < 256));
+  return std::min(bs, small ? kRowsSmallBatch : kRowsBatch);
+}
 size_t bwd_rows_smem(int ch, int bs, int bb) {
   const size_t ns = static_cast<size_t>(ch + 6) | 1;
   const size_t acc = (static_cast<size_t>(bb) * ns + 1) / 2 * 16;
@@ -2437,10 +2470,12 @@ static int rasterize_bwd_impl(const float* means2d, const float* conics, const f
   const unsigned nb = static_cast<unsigned>(n_total);
   // one block per tile (block b: the tile of rank b in the heavy-first order)
   //
-  // Records in lanes wherever that kernel applies: staged colours, sums of
-  // signed gradients only
-  if (ch >= 1 && !v_means2d_abs && rows_kernels_apply(tile_size, image_width, image_height)) {
-    const int bb = bwd_rows_batch(bs, n_total);
+  // Records in lanes where that kernel applies (staged colours, sums of signed
+  // gradients only) and is the faster one
+  const int64_t per_tile = n_isects / n_total;
+  if (ch >= 1 && !v_means2d_abs && rows_kernels_apply(tile_size, image_width, image_height) &&
+      bwd_rows_faster(tile_size, ch, n_total, per_tile)) {
+    const int bb = bwd_rows_batch(tile_size, bs, ch, n_total, per_tile);
     const size_t sm = bwd_rows_smem(ch, bs, bb);
 #define GSPLAT_BWD_ROWS(C)                                                                                     \
   raster_bwd_rows_kernel<C><<<nb, bs, sm, s>>>(a, bb, n_total, order, cost, render_alphas, last_ids,           \

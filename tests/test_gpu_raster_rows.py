@@ -235,3 +235,38 @@ def test_kernels_for_short_and_long_lists_agree(oracle, ts, C, W, H, pads):
         for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
             assert (b[k][:, n] == 0).all(), k
             assert_close_rel(host(b[k][:, :n]), host(bwd[0][k]), GRAD_RTOL, k)
+
+
+@pytest.mark.parametrize("C", [3, 4])
+@pytest.mark.parametrize("n", [129, 200, 255, 257, 529])
+def test_batches_of_many_tiles(oracle, n, C):
+    """1100 copies of one tile's image: batches of 128 entries (lists below 256,
+    and four channels) and of 256, with records that touch some of a tile's
+    waves only, so that part-filled groups carry over. Every copy's gradients
+    are the single image's, which the oracle's confirm."""
+    import torch
+
+    rng = np.random.default_rng(n + C)
+    s = make_scene(oracle, rng, 1, n, 16, 16, 16, C, opac=(0.006, 0.05), scale=(0.6, 2.0))
+    s["means2d"] = rng.uniform(0, 16, s["means2d"].shape).astype(np.float32)
+    s["flatten_ids"] = rng.permutation(n).astype(np.int32)
+    s["tile_offsets"] = np.zeros_like(s["tile_offsets"])
+    _check(oracle, s, 16, 16, 16, rng)
+    g = gsplat()
+    one = _raster_inputs(s)
+    copies = 1100
+    many = {k: v.repeat(copies, *([1] * (v.dim() - 1))) for k, v in one.items() if k != "flatten_ids"}
+    step = torch.arange(copies, device="cuda", dtype=torch.int32)
+    many["tile_offsets"] = many["tile_offsets"] + (step * n)[:, None, None]
+    many["flatten_ids"] = (one["flatten_ids"][None] + (step * n)[:, None]).reshape(-1).contiguous()
+    cot = [dev(rng.normal(size=(1, 16, 16, c)).astype(np.float32)) for c in (C, 1)]
+    out = []
+    for inp, k in ((one, 1), (many, copies)):
+        f = g.rasterize_to_pixels_3dgs_forward(inp, 16, 16, 16)
+        out.append(g.rasterize_to_pixels_3dgs_backward(
+            inp, {"render_alphas": f["render_alphas"], "last_ids": f["last_ids"]},
+            {"v_render_colors": cot[0].repeat(k, 1, 1, 1), "v_render_alphas": cot[1].repeat(k, 1, 1, 1)}, 16, 16, 16))
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        # one tile per image: each sum is rounded once per batch, whatever the batches
+        a, b = host(out[1][k]), host(out[0][k])
+        assert_close_rel(a, np.broadcast_to(b, a.shape), 1e-5, k)
