@@ -29,9 +29,9 @@
 //     the scatter left: one distribution over the range of the depth bits and
 //     a count within each bin. A tile whose depths crowd a bin takes a stable
 //     LSD radix sort on the depth bits instead, 8 bits a pass (passes whose
-//     digit is the same for the whole tile are skipped), sorted again on the
-//     id bytes and the depth bits where depths are equal. The block writes the
-//     64-bit ids and the flatten ids.
+//     digit is the same for the whole tile are skipped), and equal depths there
+//     an insertion sort (short runs) or passes on the id bytes. The block writes
+//     the 64-bit ids and the flatten ids.
 //     Short lists are sorted by one launch over every list, each longer
 //     class by a launch of a larger instantiation; lists longer than the
 //     LDS holds (kBucketMaxList) are split by their most significant varying
@@ -871,10 +871,45 @@ struct TileSorter {
   }
 };
 
+// A list's elements from the registers of distribute to LDS in list order, for
+// the radix passes, and in bits the OR and AND of its keys and of its ids. Enter
+// behind a barrier after the last read of kv and bits.
+template <int B, int ITEMS>
+__device__ __forceinline__ void stage_radix(const uint2 (&e)[ITEMS], int n, uint2* s_kv, uint32_t* s_bits) {
+  const int t = threadIdx.x;
+  if (t < 4) s_bits[t] = (t & 1) ? ~0u : 0u;
+  __syncthreads();
+  uint32_t ko = 0u, ka = ~0u, vo = 0u, va = ~0u;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int j = r * B + t;
+    if (j < n) {
+      s_kv[j] = e[r];
+      ko |= e[r].x;
+      ka &= e[r].x;
+      vo |= e[r].y;
+      va &= e[r].y;
+    }
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    ko |= __shfl_xor(ko, off, kWave);
+    ka &= __shfl_xor(ka, off, kWave);
+    vo |= __shfl_xor(vo, off, kWave);
+    va &= __shfl_xor(va, off, kWave);
+  }
+  if (t % kWave == 0) {
+    atomicOr(&s_bits[0], ko);
+    atomicAnd(&s_bits[1], ka);
+    atomicOr(&s_bits[2], vo);
+    atomicAnd(&s_bits[3], va);
+  }
+  __syncthreads();
+}
+
 // One-distribution sort of the n pairs at src (n <= B * ITEMS), written as
-// sort_range below; false, with nothing written, when a bin is crowded. False
-// comes behind a barrier after every read of the shared arrays, so the caller
-// may write them at once.
+// sort_range below; false, with nothing written and the list staged for the
+// radix passes, when a bin is crowded.
 //
 // The bins divide the keys' range evenly (8 per thread, two 16-bit counts a
 // word): they are counted by LDS atomics, their exclusive scan gives the bins'
@@ -888,7 +923,16 @@ struct TileSorter {
 //
 // Threads past the list count in words of their own, without a branch, so that
 // the atomics of a thread's elements overlap.
+//
+// Counting a crowded bin is a chain of atomics on one word, so a wave that finds
+// kSampleCrowd of its first 64 elements in the bin of the first or of the 33rd
+// (which then holds about a quarter of the list) gives up before it counts. The
+// radix passes then start from the registers. 3969 lists of 1240 entries, against
+// radix passes at once: even depths 33 us (65), one depth 51 (67), four 118
+// (120), 98% within 1/3000 of the range 76.5 (76). Where the distribution fails
+// late it costs up to a tenth (98% within 1/500, 600 entries: 54 us, 49).
 constexpr int kBinCrowd = 48;
+constexpr int kSampleCrowd = 16;
 
 template <int B, int ITEMS>
 __device__ __forceinline__ bool distribute(const uint2* src, int n, uint64_t hi, int64_t* out_ids, int32_t* out_flat,
@@ -929,18 +973,26 @@ __device__ __forceinline__ bool distribute(const uint2* src, int n, uint64_t hi,
   const uint32_t span = s_bits[0] - lowest;
   if (span == 0 && n > kBinCrowd) {  // one depth: the radix sort on the ids
     __syncthreads();                 // every wave has read s_bits
+    stage_radix<B, ITEMS>(e, n, s_kv, s_bits);
     return false;
   }
   const int shift = max(0, (32 - __builtin_clz(span | 1u)) - (31 - __builtin_clz(static_cast<unsigned>(kBins))));
   auto bin_of = [&](uint32_t key) { return (key - lowest) >> shift; };
   auto bin_word = [&](int r, uint32_t b) { return r * B + t < n ? s_bins + (b >> 1) : s_dstart + 64 + lane; };
+  bool crowded = false;
+  if (n > kBinCrowd * kWave / kSampleCrowd && wave * kWave + kWave <= n) {  // wave-uniform
+    const int b = static_cast<int>(bin_of(e[0].x));
+    crowded = __popcll(__ballot(b == __builtin_amdgcn_readlane(b, 0))) >= kSampleCrowd ||
+              __popcll(__ballot(b == __builtin_amdgcn_readlane(b, 32))) >= kSampleCrowd;
+  }
+  if (!crowded) {
 #pragma unroll
-  for (int r = 0; r < ITEMS; ++r) {
-    const uint32_t b = bin_of(e[r].x);
-    atomicAdd(bin_word(r, b), 1u << ((b & 1u) * 16u));
+    for (int r = 0; r < ITEMS; ++r) {
+      const uint32_t b = bin_of(e[r].x);
+      atomicAdd(bin_word(r, b), 1u << ((b & 1u) * 16u));
+    }
   }
   __syncthreads();
-  bool crowded = false;
   uint32_t c[kBinWords], sum = 0;
 #pragma unroll
   for (int q = 0; q < kBinWords; ++q) {
@@ -951,7 +1003,10 @@ __device__ __forceinline__ bool distribute(const uint2* src, int n, uint64_t hi,
   }
   const uint32_t inc = static_cast<uint32_t>(wave_inclusive_scan(static_cast<int>(sum)));
   if (lane == kWave - 1) s_dstart[wave] = inc;
-  if (__syncthreads_or(crowded)) return false;
+  if (__syncthreads_or(crowded)) {
+    stage_radix<B, ITEMS>(e, n, s_kv, s_bits);
+    return false;
+  }
   uint32_t run = inc - sum;
 #pragma unroll
   for (int w = 0; w < W; ++w) run += w < wave ? s_dstart[w] : 0u;
@@ -1007,50 +1062,14 @@ __device__ __forceinline__ void sort_range(const uint2* src, int64_t len, uint64
   } else {
     if (distribute<B, ITEMS>(src, n, hi, out_ids, out_flat, s_kv, s_wcnt, s_dstart, s_bits)) return;
   }
-  // Depths of very uneven spread or many equal ones: radix passes.
-  if (t < 4) s_bits[t] = (t & 1) ? ~0u : 0u;
-  __syncthreads();
-  // the bits that vary over the list: passes on digits every element shares
-  // are skipped. The list is loaded ITEMS elements per thread, all loads in
-  // flight before the first LDS store (lists this sort holds have at most
-  // B * ITEMS elements).
-  uint32_t ko = 0u, ka = ~0u, vo = 0u, va = ~0u;
-  {
-    uint2 e[ITEMS];
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-      const int j = r * B + t;
-      e[r] = j < n ? src[j] : make_uint2(0u, ~0u);
-    }
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-      const int j = r * B + t;
-      if (j < n) {
-        s_kv[j] = e[r];
-        ko |= e[r].x;
-        ka &= e[r].x;
-        vo |= e[r].y;
-        va &= e[r].y;
-      }
-    }
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    ko |= __shfl_xor(ko, off, kWave);
-    ka &= __shfl_xor(ka, off, kWave);
-    vo |= __shfl_xor(vo, off, kWave);
-    va &= __shfl_xor(va, off, kWave);
-  }
-  if (t % kWave == 0) {
-    atomicOr(&s_bits[0], ko);
-    atomicAnd(&s_bits[1], ka);
-    atomicOr(&s_bits[2], vo);
-    atomicAnd(&s_bits[3], va);
-  }
-  __syncthreads();
+  // Depths of very uneven spread or many equal ones: radix passes (passes on
+  // digits that every element shares are skipped).
   const uint32_t kvary = s_bits[0] ^ s_bits[1], ivary = s_bits[2] ^ s_bits[3];
   S srt{s_kv, s_wcnt, s_dstart, n, (n + S::W * kWave - 1) / (S::W * kWave)};
-  if (n > 1) {
+  if (kvary == 0) {  // one depth: by flatten id
+#pragma unroll 1
+    for (int shift = 0; shift < 32; shift += 8) srt.pass(true, shift, (ivary >> shift) & 255u);
+  } else {
 #pragma unroll 1
     for (int shift = 0; shift < 32; shift += 8) srt.pass(false, shift, (kvary >> shift) & 255u);
     // equal depths: their entries go in flatten-id order. A run of up to
@@ -1140,10 +1159,9 @@ struct TileSortLds {
   uint32_t bits[4];  // OR and AND of the keys, OR and AND of the ids
 };
 
-// Waves per SIMD that the LDS admits: the register budget of the sorts. What
-// that budget spills is the radix passes' arrays, off the usual path (4346
-// lists of 1241 entries on average: 50 us at four waves per SIMD, 44 at five,
-// 40 at six).
+// Waves per SIMD that the LDS admits: the register budget of the sorts, at which
+// none of them spills (4346 lists of 1241 entries on average: 50 us at four waves
+// per SIMD, 44 at five, 40 at six).
 constexpr int tile_sort_waves(int b, int items) {
   return static_cast<int>(kLdsBytes / (b * items * 8 + b / kWave * 1024 + 1040)) * b / kWave / 4;
 }
