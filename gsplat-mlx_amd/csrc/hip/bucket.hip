@@ -508,8 +508,10 @@ __device__ void grid_prefix_2d(int32_t* g, int tw, int th, int nthreads) {
 // total grids weighted by the tiles each grid point covers, (tw - x)(th - y),
 // so no block waits for another. One block for all images took 7 to 12 us an
 // image: 94.7 -> 32.3 us over 8 images of 8160 tiles, 13.7 -> 10.3 us over the 2
-// images of a 200k-Gaussian list build; one image took 8.0 and takes 8.2.
-constexpr int kTilePassImages = 32;
+// images of a 200k-Gaussian list build; one image took 8.0 and takes 8.2. The sums
+// grow with the square of the images: with the block scan, 33 images of 8160
+// tiles 419 -> 135 us, 256 3187 -> 801, 1000 12.5 -> 7.5 ms (of 9 tiles 1.5 -> 0.23).
+constexpr int kTilePassImages = 1024;
 
 __global__ void __launch_bounds__(kTilePassBlock) bucket_tile_pass_kernel(BucketDims d,
                                                                           const int32_t* __restrict__ totals,

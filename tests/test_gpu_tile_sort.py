@@ -69,13 +69,13 @@ def test_a_frame_of_one_depth(per_tile, side, planes):
     np.testing.assert_array_equal(host(out["tile_offsets"]).ravel(), np.cumsum(lengths) - lengths)
 
 
-@pytest.mark.parametrize("images", [1, 2, 7, 32, 33])
+@pytest.mark.parametrize("images", [1, 2, 7, 32, 33, 1024, 1025])
 def test_images_start_after_the_earlier_ones(images):
     """Offsets and lists over several images (a tile pass block per image up to
-    32 of them, one block for all beyond), one image empty, against a numpy
+    1024 of them, one block for all beyond), one image empty, against a numpy
     enumeration."""
     rng = np.random.default_rng(images)
-    n, tw, th = 300, 5, 3
+    n, tw, th = 300 if images < 100 else 7, 5, 3
     m = rng.uniform(-10, 90, (images, n, 2)).astype(np.float32)
     r = rng.integers(0, 30, (images, n, 2)).astype(np.int32)
     if images > 1:
@@ -83,8 +83,9 @@ def test_images_start_after_the_earlier_ones(images):
     d = rng.uniform(0.2, 9.0, (images, n)).astype(np.float32)
     g = gsplat()
     out = g.intersect_tile_offsets_forward({"means2d": dev(m), "radii": dev(r), "depths": dev(d)}, images, 16, tw, th)
-    lo = np.clip(np.floor((m - r) / 16), 0, [tw, th]).astype(int)
-    hi = np.clip(np.ceil((m + r) / 16), 0, [tw, th]).astype(int)
+    rf = r.astype(np.float32)  # the operator's float32 sums: a float64 m - r can fall on the other side of a tile edge
+    lo = np.clip(np.floor((m - rf) / 16), 0, [tw, th]).astype(int)
+    hi = np.clip(np.ceil((m + rf) / 16), 0, [tw, th]).astype(int)
     rows = []
     for i in range(images):
         for k in range(n):
