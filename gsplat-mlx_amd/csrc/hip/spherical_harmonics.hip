@@ -1017,8 +1017,8 @@ int launch_cam_bwd(const float* means, const float* viewmats, const float* dc, c
                                       s);
 }
 
-// The operator's kernels for rows of exactly the active bases (K == A) at
-// 16-byte aligned pointers: a wave per 64 rows. The rows are one contiguous
+// The operator's kernels for rows of exactly the active bases (K == A, degree 1
+// and up) at 16-byte aligned pointers: a wave per 64 rows. The rows are one contiguous
 // span, copied to LDS and (the backward's gradient rows, over the coefficients)
 // back with 16-byte accesses whose row and column split is a constant one, and
 // each lane reads and writes its own row there. Row strides: whole float4s
@@ -1027,7 +1027,11 @@ int launch_cam_bwd(const float* means, const float* viewmats, const float* dc, c
 //
 // The general kernels split every float's index with a multiply and form each
 // gradient value from LDS at the store. 600,011 rows of degree 3: forward
-// 36 -> 23 us, backward 66 -> 42 us (5.7 and 6.0 TB/s).
+// 35 -> 23 us, backward 64 -> 42 us with the inputs in the last-level cache from
+// the call before; with other coefficients each call 46 -> 26 and 84 -> 43 us.
+// 2,000,000 rows, more than that cache holds: 128 -> 80 and 270 -> 154 us (5.4
+// TB/s). Degree 0 stays with the general kernels: three floats a row are as fast
+// there (1,200,000 rows forward: 8.2 us, 8.8 here).
 constexpr int kShRows = kWave;
 
 template <int DEG>
@@ -1152,11 +1156,11 @@ __global__ void __launch_bounds__(kShRows) sh_rows_bwd_kernel(const float* __res
     }
   }
   float* row = rows + t * R::PW;
-  if (DEG >= 1 && v_dirs) rows_to_lds<DEG>(rows, coeffs + e0 * R::W, cnt);
+  if (v_dirs) rows_to_lds<DEG>(rows, coeffs + e0 * R::W, cnt);
   __syncthreads();
   if (in && v_dirs) {
     float vd[3] = {0.0f, 0.0f, 0.0f};
-    if (on && DEG >= 1) {
+    if (on) {
       float co[R::W];
       row_read<DEG>(row, co);
       sh_dir_vjp<DEG>(d, co, vc, vd);
@@ -1196,11 +1200,14 @@ int launch_fwd(const float* dirs, const float* coeffs, const uint8_t* masks, int
                hipStream_t s) {
   {
     KernelTimer timer("sh_fwd", s);
-    if (whole_rows(DEG, K, coeffs, nullptr))
-      sh_rows_fwd_kernel<DEG><<<grid_for(n, kShRows), kShRows, 0, s>>>(dirs, coeffs, masks, n, colors);
-    else
-      sh_fwd_kernel<DEG><<<grid_for(n, kShBlock), kShBlock, 0, s>>>(dirs, coeffs, masks, n, K,
-                                                                    magic_for(static_cast<uint32_t>(K * 3)), colors);
+    if constexpr (DEG >= 1) {
+      if (whole_rows(DEG, K, coeffs, nullptr)) {
+        sh_rows_fwd_kernel<DEG><<<grid_for(n, kShRows), kShRows, 0, s>>>(dirs, coeffs, masks, n, colors);
+        return check_launch("spherical_harmonics_forward");
+      }
+    }
+    sh_fwd_kernel<DEG><<<grid_for(n, kShBlock), kShBlock, 0, s>>>(dirs, coeffs, masks, n, K,
+                                                                  magic_for(static_cast<uint32_t>(K * 3)), colors);
   }
   return check_launch("spherical_harmonics_forward");
 }
@@ -1210,13 +1217,16 @@ int launch_bwd(const float* dirs, const float* coeffs, const uint8_t* masks, con
                int64_t K, float* v_dirs, float* v_coeffs, hipStream_t s) {
   {
     KernelTimer timer("sh_bwd", s);
-    if (whole_rows(DEG, K, coeffs, v_coeffs))
-      sh_rows_bwd_kernel<DEG><<<grid_for(n, kShRows), kShRows, 0, s>>>(dirs, coeffs, masks, v_colors, n, v_dirs,
-                                                                       v_coeffs);
-    else
-      sh_bwd_kernel<DEG><<<grid_for(n, kShBlock), kShBlock, 0, s>>>(dirs, coeffs, masks, v_colors, n, K,
-                                                                 magic_for(static_cast<uint32_t>(K * 3)), v_dirs,
-                                                                 v_coeffs);
+    if constexpr (DEG >= 1) {
+      if (whole_rows(DEG, K, coeffs, v_coeffs)) {
+        sh_rows_bwd_kernel<DEG><<<grid_for(n, kShRows), kShRows, 0, s>>>(dirs, coeffs, masks, v_colors, n, v_dirs,
+                                                                         v_coeffs);
+        return check_launch("spherical_harmonics_backward");
+      }
+    }
+    sh_bwd_kernel<DEG><<<grid_for(n, kShBlock), kShBlock, 0, s>>>(dirs, coeffs, masks, v_colors, n, K,
+                                                                  magic_for(static_cast<uint32_t>(K * 3)), v_dirs,
+                                                                  v_coeffs);
   }
   return check_launch("spherical_harmonics_backward");
 }

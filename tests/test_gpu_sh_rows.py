@@ -1,8 +1,9 @@
 """The spherical harmonics operator on rows of exactly the active bases (whole
-float4s per row at degrees 1 and 3, odd row lengths at 0, 2 and 4): the same
-bits as on the leading bases of longer rows, which take the general kernels,
-for whole and partial blocks of 64 rows, masks, and with and without direction
-gradients; and views whose rows are not 16-byte aligned."""
+float4s per row at degrees 1 and 3, odd row lengths at 2 and 4; degree 0 has
+the general kernels only): the same bits as on the leading bases of longer
+rows, which take the general kernels, for whole and partial blocks of 64 rows,
+masks, and with and without direction gradients; and views whose rows are not
+16-byte aligned."""
 import numpy as np
 import pytest
 
