@@ -128,7 +128,9 @@ __device__ __forceinline__ float exp_alpha(float y) {
   return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
 }
 
-// exp_alpha for y in (-2.98e9, 0], bit for bit, without the lower clamp.
+// exp_alpha for y in (-1.48e9, 0] without the lower clamp: the same bits down to
+// -103, and below that at most 2^-149 as well, which no alpha test passes. The
+// conversion of n bounds the range (|n| < 2^31).
 __device__ __forceinline__ float exp_alpha_bounded(float y) {
   const float head = 1.44269502162933349609375f;  // float(log2 e)
   const float tail = __uint_as_float(0x32a5705fu);
@@ -145,9 +147,10 @@ __device__ __forceinline__ float exp_alpha_bounded(float y) {
 // - kGeneralRecord clear: a conic well inside the positive definite ones
 //   (det > 1e-4 c0 c2 keeps the computed sigma >= 0: its rounding is below
 //   1e-6 of c0 dx^2 + c2 dy^2, the form above 5e-5 of it, and neither
-//   underflows), and an opacity up to 1. A visiting wave has a pixel with
-//   sigma below 6 within 44 pixels of every other one, and c0 + c2 <= 2e6
-//   then keeps sigma below 2e9, so the exponential needs no clamp.
+//   underflows), and an opacity up to 1. A visiting wave's 8x8 pixels have a
+//   point with sigma below 6 within 9.9 of every pixel; sqrt(sigma) is a norm of
+//   the offset, at most sqrt((c0 + c2) / 2) <= 1000 per pixel, so sigma stays below
+//   (2.5 + 9900)^2 < 1e8 and the exponential needs no clamp.
 // - kCappedRecord clear: also an opacity up to 0.99, so alpha = o exp(-sigma)
 //   never meets the cap.
 // - kNonFiniteRecord: a non-finite staged colour, in the backward also a
@@ -1310,7 +1313,7 @@ __device__ __forceinline__ void row16_sum4(float (&v)[4], float (&before)[4]) {
 // - Groups without capped or general records (see above) skip the cap's and
 //   sigma's tests.
 // - The waves add their sums to one slot per entry in double (LDS atomics), so
-//   the order in which waves arrive does not show in the rounded result.
+//   the order in which waves arrive hardly ever shows in the rounded result.
 //
 // - While entries remain before a batch, a wave evaluates whole groups only;
 //   the next batch starts at the first entry some wave left over (each wave
