@@ -1715,6 +1715,7 @@ __global__ void __launch_bounds__(576) __attribute__((amdgpu_waves_per_eu(4))) r
         }
       }
       if (g0 == 0) load_records(b1n, b0n);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the pixels' state: lane 15 wrote it, lane 0 reads it next
     }
     __syncthreads();
     __builtin_amdgcn_s_waitcnt(kWaitVmemOnly);
