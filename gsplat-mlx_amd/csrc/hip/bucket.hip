@@ -13,7 +13,7 @@
 //     its grid, and tiles_per_gauss is written here;
 //  2. block scan: per grid point, the exclusive sum of the grids of the
 //     image's earlier blocks (in place) and the image total;
-//  3. tile pass (one block): the 2D inclusive prefix of an image's total grid
+//  3. tile pass (a block per image): the 2D inclusive prefix of its total grid
 //     is every tile's entry count; their exclusive scan is each tile's first
 //     slot (the reference's tile offsets), the total M and the largest count;
 //     lists too long for the smallest tile sort are binned by length class;
@@ -931,8 +931,8 @@ __device__ __forceinline__ void stage_radix(const uint2 (&e)[ITEMS], int n, uint
 // (which then holds about a quarter of the list) gives up before it counts. The
 // radix passes then start from the registers. 3969 lists of 1240 entries, against
 // radix passes at once: even depths 33 us (65), one depth 51 (67), four 118
-// (120), 98% within 1/3000 of the range 76.5 (76). Where the distribution fails
-// late it costs up to a tenth (98% within 1/500, 600 entries: 54 us, 49).
+// (120), 98% within 1/1700 of the bits' range 76.5 (76). Where the distribution
+// fails late it costs up to a tenth (98% within 1/115, 600 entries: 54 us, 49).
 constexpr int kBinCrowd = 48;
 constexpr int kSampleCrowd = 16;
 
