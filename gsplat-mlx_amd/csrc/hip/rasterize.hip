@@ -2123,17 +2123,19 @@ size_t fwd_rows_smem(int ch, int n_waves, int pixels, int bb) {
 // rectangles and record lists, in the kernel's order.
 // Batches: 256 entries leave the fewest barriers and flushes (1M Gaussians, 4346
 // tiles of 1245 entries: 232 us against 242 at 128). Of side 16, 128 keep as many
-// blocks resident (by registers, 4 per CU) and suit shorter lists: 1.0 to 1.16
-// times the speed of 256 at 70 to 250 entries per tile, 0.86 to 1.0 from 270 on.
-// With four channels LDS admits 3 blocks of 256 entries or 4 of 128: 1.0 to 1.2
-// times the speed.
+// blocks resident (by registers, 4 on each of 256 CUs) and suit shorter lists, the
+// more the fewer rounds of resident blocks there are. Time of 256 over that of
+// 128: 1.0-1.18 at 1900 to 5700 tiles and 70 to 260 entries per tile (one scene
+// 0.9), 0.93-1.1 at 320; at 7500 to 41,000 tiles 0.98-1.1 at 70 to 110, 0.93-1.05 at
+// 140 to 180, 0.92-1.0 beyond. With four channels LDS admits 3 blocks of 256
+// entries or 4 of 128: 1.0-1.2.
 // Up to 1024 tiles 128, though 256 are 1.0 to 1.3 times as fast there (side 24
 // up to 1.4): tiles add to a Gaussian by float atomics, in no fixed order, and
 // with 256 entries this showed more. 10,000 Gaussians at 256x256: three quaternion
 // gradients of one Gaussian, all cancellation, differed by 3e-4 between a third
 // of 120 runs; with 128 none by 1e-4.
 int bwd_rows_batch(int ts, int bs, int ch, int64_t n_tiles, int64_t per_tile) {
-  const bool small = n_tiles <= 1024 || (ts == 16 && (ch == 4 || per_tile < 256));
+  const bool small = n_tiles <= 1024 || (ts == 16 && (ch == 4 || per_tile < (n_tiles <= 6144 ? 256 : 160)));
   return std::min(bs, small ? kRowsSmallBatch : kRowsBatch);
 }
 size_t bwd_rows_smem(int ch, int bs, int bb) {

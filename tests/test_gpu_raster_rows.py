@@ -1,13 +1,15 @@
 """The rasterizer kernels with records in lanes (tile sides 8, 16 and 24, one to
-four channels, no absolute gradients) against the oracle, where their groups of
-16 records, their batches of 128 and 256 entries, their record classes and the
-forward's pixel blocks meet: list lengths around 16, 128 and 256, every tile
-side, opacities over the 0.99 cap, ill-conditioned conics, opacities over 1,
-non-finite records, and grids on both sides of the forward's block sizes.
+four channels, no absolute gradients, lists long enough) against the oracle,
+where their groups of 16 records, their batches of 128 and 256 entries, their
+record classes and the forward's pixel blocks meet: list lengths around 16, 128
+and 256 (the shortest take the kernels with pixels in lanes), every tile side,
+opacities over the 0.99 cap, ill-conditioned conics, opacities over 1,
+non-finite and overflowing values, and grids on both sides of the forward's
+block sizes, of the backward's batches and of the rules that choose the kernel.
 
-Tolerance: images 1e-4 and exact last contributors as elsewhere; the gradients' usual bar, 1e-3 of each element or of 1% of the
-tensor's largest (both sides round every pixel's terms in float32; the sums
-run in another order).
+Tolerance: images 1e-4 and exact last contributors as elsewhere; the gradients'
+usual bar, 1e-3 of each element or of 1% of the tensor's largest (both sides
+round every pixel's terms in float32; the sums run in another order).
 """
 import numpy as np
 import pytest
@@ -240,8 +242,8 @@ def test_kernels_for_short_and_long_lists_agree(oracle, ts, C, W, H, pads):
 @pytest.mark.parametrize("C", [3, 4])
 @pytest.mark.parametrize("n", [129, 200, 255, 257, 529])
 def test_batches_of_many_tiles(oracle, n, C):
-    """1100 copies of one tile's image: batches of 128 entries (lists below 256,
-    and four channels) and of 256, with records that touch some of a tile's
+    """1100 copies of one tile's image: batches of 128 entries (lists below 256 on
+    such a grid, and four channels) and of 256, with records that touch some of a tile's
     waves only, so that part-filled groups carry over. Every copy's gradients
     are the single image's, which the oracle's confirm."""
     import torch
